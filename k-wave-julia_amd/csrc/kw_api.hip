@@ -1455,8 +1455,8 @@ class Batch final : public BatchBase {
     for (hipEvent_t e : done_)
       if (e) (void)hipEventDestroy(e);
     if (tick_ev_) (void)hipEventDestroy(tick_ev_);
-    for (hipStream_t l : lanes_)
-      if (l) (void)hipStreamDestroy(l);
+    for (size_t l = 1; l < lanes_.size(); ++l)   // lanes_[0] is stream_
+      if (lanes_[l]) (void)hipStreamDestroy(lanes_[l]);
     if (stream_) (void)hipStreamDestroy(stream_);
   }
   void run(long long n) override {
