@@ -285,7 +285,9 @@ int32_t kw_sim_destroy(kw_sim* sim);
  * reference runs one simulation per call).  Every pass is one launch per
  * line length over all simulations, the step index lives on the device and,
  * with KW_BATCH_GRAPH in use_graph (a flags word; 0 and 1 keep their old
- * meaning), one step is captured in a hipGraph and replayed.  With
+ * meaning), a step whose passes form one chain (simulations of one grid
+ * size) is captured in a hipGraph and replayed; chains of several line
+ * lengths run beside each other on streams.  With
  * KW_BATCH_PERSISTENT each batched pass runs as a persistent grid (as many
  * workgroups as fit the device at once, each looping over the pass's
  * workgroup tiles) instead of one workgroup per tile; KW_BATCH_GRID8(n)

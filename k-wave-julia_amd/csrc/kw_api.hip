@@ -1462,7 +1462,11 @@ class Batch final : public BatchBase {
   void run(long long n) override {
     HIPC(hipSetDevice(dev_));
     for (long long i = 0; i < n && t_ < Nt_; ++i) {
-      if (use_graph_) {
+      // Only a step of one chain is captured: replaying a graph with several
+      // branches has ended in a host segmentation fault inside the runtime
+      // (for some branch shapes, on its first replays), so a step whose groups
+      // run on several lanes is enqueued on them each time.
+      if (use_graph_ && lanes_.size() == 1) {
         if (!exec_) capture();
         HIPC(hipGraphLaunch(exec_, stream_));
       } else {
