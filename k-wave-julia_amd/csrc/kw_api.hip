@@ -291,7 +291,8 @@ class Sim final : public SimBase {
     if (stokes_) raise(KW_ERR_UNSUPPORTED, "the c0 gradient needs the heterogeneous equation-of-state branch");
     if (maps_f16_) raise(KW_ERR_UNSUPPORTED, "the c0 gradient needs maps in the kernel precision");
     for (int a = 0; a < nd_; ++a)
-      if (bs_[a]) raise(KW_ERR_UNSUPPORTED, "the c0 gradient needs axis lengths with a compiled line-FFT plan");
+      if (!size_supported(N_[a]))
+        raise(KW_ERR_UNSUPPORTED, "the c0 gradient needs axis lengths with a compiled line-FFT plan");
     if (tr_ || (psrc_[0].any && p_dir_)) raise(KW_ERR_UNSUPPORTED, "time reversal / Dirichlet sources");
     for (int a = 0; a < nd_; ++a)
       if (usrc_[a].any && u_dir_) raise(KW_ERR_UNSUPPORTED, "Dirichlet velocity sources");
@@ -380,6 +381,7 @@ class Sim final : public SimBase {
       A.So = pa_[a].So;
       A.n_lines = pa_[a].n_lines;
       A.x_blocks = pa_[a].x_blocks;
+      A.swz = pa_[a].swz;
     }
     // ---- reverse sweep over segments
     for (long long s = nseg - 1; s >= 0; --s) {
@@ -415,7 +417,7 @@ class Sim final : public SimBase {
         for (int a = 0; a < nd_; ++a) {
           aa[a].accumulate = a > 0 ? 1 : 0;
           HIPC(launch_adj_pass<T>(cfg_[a].n, a == 0, cfg_[a].grid, cfg_[a].block, cfg_[a].shmem, stream_, aa[a],
-                                  cfg_[a].pv));
+                                  cfg_[a].family()));
         }
       }
     }
@@ -465,22 +467,22 @@ class Sim final : public SimBase {
       SpecArgs<T> Y = sa_[0];
       Y.mode = 0;
       Y.S2 = nullptr;
-      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].pv));
+      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].family()));
       SpecArgs<T> Z = sa_[1];
       Z.mode = 5;
       Z.S2 = S2_.as<Cx<T>>();
       Z.M2 = M2;
-      HIPC(launch_spec<T>(spec_[1].n, spec_[1].grid, spec_[1].block, spec_[1].shmem, stream_, Z, spec_[1].pv));
+      HIPC(launch_spec<T>(spec_[1].n, spec_[1].grid, spec_[1].block, spec_[1].shmem, stream_, Z, spec_[1].family()));
       Y.mode = 1;
-      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].pv));
+      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].family()));
       Y.S1 = S2_.as<Cx<T>>();
-      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].pv));
+      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].family()));
     } else if (nd_ == 2) {
       SpecArgs<T> Y = sa_[0];
       Y.mode = 5;
       Y.S2 = S2_.as<Cx<T>>();
       Y.M2 = M2;
-      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].pv));
+      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].family()));
     }
     C2RArgs<T> c = ca_;
     c.S2 = nullptr;
@@ -578,15 +580,15 @@ class Sim final : public SimBase {
     }
     for (int a = 0; a < nd_; ++a) {
       if (N_[a] < 1) raise(KW_ERR_INVALID, "grid size must be positive");
-      // compiled plan, or a chirp-z (Bluestein) line on a power-of-two plan
-      bs_[a] = !size_supported(N_[a]);
+      // compiled plan, or a chirp-z (Bluestein) line on a longer plan
+      if (!size_supported(N_[a]) && batch_mode_)
+        raise(KW_ERR_UNSUPPORTED, "axis length " + std::to_string(N_[a]) +
+                                      " has no compiled plan; batches take compiled lengths only");
+      bs_[a] = !size_supported(N_[a]) && !direct_size(N_[a]);
       M_[a] = bs_[a] ? bluestein_plan(N_[a]) : N_[a];
       if (M_[a] == 0)
         raise(KW_ERR_UNSUPPORTED, "axis length " + std::to_string(N_[a]) +
                                       " is longer than the largest chirp-z line (2048) and has no compiled plan");
-      if (bs_[a] && batch_mode_)
-        raise(KW_ERR_UNSUPPORTED, "axis length " + std::to_string(N_[a]) +
-                                      " has no compiled plan; batches take compiled lengths only");
       if (d.pml_size[a] < 0) raise(KW_ERR_INVALID, "pml_size must be >= 0");
       if (2LL * d.pml_size[a] > N_[a] + 0 && d.pml_size[a] > N_[a])
         raise(KW_ERR_INVALID, "pml_size larger than the grid");
@@ -607,6 +609,8 @@ class Sim final : public SimBase {
     }
     nvox_ = N_[0] * N_[1] * N_[2];
     plane_ = nvox_ / nfire_;
+    // p, u_d, rho_d, two maps and the half spectrum; a batch's launches mix grids
+    large_ = !batch_mode_ && beyond_cache(2 * nd_ + 4, nvox_, (int)sizeof(T));
     NH_ = N_[0] / 2 + 1;
     NHP_ = (NH_ + 15) / 16 * 16;  // 128-byte aligned spectrum rows (FP32)
     dt_ = d.dt;
@@ -699,16 +703,16 @@ class Sim final : public SimBase {
   PassCfg pass_cfg(long long n, bool contig, long long lines, long long outer, int cls, bool bs = false) {
     PassCfg c;
     c.n = (int)n;
-    // plan family: 0 strided, 1 contiguous, 2 complex-to-real, 4 contiguous chirp-z lines, or a tuned
-    // alternative (single simulations on compiled lengths; batch kernels take the defaults)
-    const int dflt_v = contig && bs ? 4 : (cls == TC_C2R ? 2 : (contig ? 1 : 0));
+    // plan family: the pass's default, or a tuned alternative (single simulations on compiled lengths;
+    // batch kernels take the defaults)
+    const int dflt_v = default_family<T>(cls == TC_C2R ? kC2R : (contig ? kContig : kStrided), contig && bs);
     c.pv = (bs || batch_mode_) ? -1 : tuned_plan((int)sizeof(T), cls, (int)n);
     if (c.pv == dflt_v) c.pv = -1;   // the default family: its own kernels
-    const int tpl = plan_tpl((int)n, c.pv >= 0 ? c.pv : dflt_v);
+    c.wide = sizeof(T) == 4 && !contig && !bs && large_ && wide_strided((int)n) && (N_[0] * sizeof(T)) % 128 == 0 &&
+             c.pv < 0;
+    const int tpl = plan_tpl((int)n, c.wide ? kWideFamily : (c.pv >= 0 ? c.pv : dflt_v));
     const size_t line_bytes = (size_t)plan_pitch((int)n) * sizeof(Cx<T>);
-    // strided lines: at least 16 line pairs per workgroup (128-byte rows in FP32)
-    // when that fits 512 threads; contiguous lines: 256 threads
-    int lpw = (contig ? 256 : std::max(256, std::min(512, 16 * tpl))) / tpl;
+    int lpw = contig ? contig_lines(tpl) : strided_lines(tpl, sizeof(T), large_);
     while (lpw > 1 && (size_t)lpw * line_bytes > lds_max_) lpw /= 2;
     int maxl = (cls == TC_C2R ? 256 : 512) / tpl;   // the kernels' launch bounds
     while (maxl > 1 && (size_t)maxl * line_bytes > lds_max_) maxl /= 2;
@@ -718,9 +722,9 @@ class Sim final : public SimBase {
     const long long pairs = (lines + 1) / 2;
     while (!batch_mode_ && lpw > 1 && lpw / 2 >= pairs) lpw /= 2;
     // small grids (2-D, few lines): fewer lines per workgroup until the launch
-    // has two workgroups per CU, keeping at least one full wave per workgroup
+    // has two workgroups per CU
     if (!batch_mode_) {
-      const int min_lpw = std::max(1, 64 / tpl);
+      const int min_lpw = min_lines(contig, tpl, sizeof(T));
       const long long o = contig ? 1 : std::max<long long>(outer, 1);
       while (lpw / 2 >= min_lpw && ((pairs + lpw - 1) / lpw) * o < fill_wgs_) lpw /= 2;
     }
@@ -741,10 +745,12 @@ class Sim final : public SimBase {
     PassCfg c;
     c.n = (int)n;
     c.pv = (bs_[cls == TC_SPEC_Y ? 1 : 2] || batch_mode_) ? -1 : tuned_plan((int)sizeof(T), cls, (int)n);
-    if (c.pv == 0) c.pv = -1;   // the default family: its own kernels
-    const int tpl = plan_tpl((int)n, c.pv >= 0 ? c.pv : 0);
+    const int dflt_v = default_family<T>(kStrided);
+    if (c.pv == dflt_v) c.pv = -1;   // the default family: its own kernels
+    c.wide = sizeof(T) == 4 && !bs_[cls == TC_SPEC_Y ? 1 : 2] && large_ && wide_spectral((int)n) && c.pv < 0;
+    const int tpl = plan_tpl((int)n, c.wide ? kWideFamily : (c.pv >= 0 ? c.pv : dflt_v));
     const size_t line_bytes = (size_t)plan_pitch((int)n) * sizeof(Cx<T>);
-    int lpw = std::max(256, std::min(512, 16 * tpl)) / tpl;   // as for strided passes
+    int lpw = strided_lines(tpl, sizeof(T), large_);   // one complex line is as wide as a pair of real ones
     while (lpw > 1 && (size_t)lpw * line_bytes > lds_max_) lpw /= 2;
     int maxl = 512 / tpl;
     while (maxl > 1 && (size_t)maxl * line_bytes > lds_max_) maxl /= 2;
@@ -752,7 +758,7 @@ class Sim final : public SimBase {
     c.req = lpw;
     while (!batch_mode_ && lpw > 1 && lpw / 2 >= NH_) lpw /= 2;
     if (!batch_mode_) {   // as in pass_cfg: fill the device on small grids
-      const int min_lpw = std::max(1, 64 / tpl);
+      const int min_lpw = min_lines(false, tpl, sizeof(T));
       while (lpw / 2 >= min_lpw && ((NH_ + lpw - 1) / lpw) * std::max<long long>(outer, 1) < fill_wgs_) lpw /= 2;
     }
     c.lpw = lpw;
@@ -993,6 +999,7 @@ class Sim final : public SimBase {
       A.ch = chirp(a);
       const PassCfg& c = cfg_[a];
       A.x_blocks = (int)(((N_[0] + 1) / 2 + c.lpw - 1) / c.lpw);
+      A.swz = a > 0 && swizzled_rows(c.lpw, sizeof(T), N_[0] * (long long)sizeof(T));
       if (a == 1) {
         A.Sa = N_[0];
         A.So = N_[0] * N_[1];
@@ -1044,6 +1051,7 @@ class Sim final : public SimBase {
       Y.Sa = NHP_;
       Y.So = NHP_ * N_[1];
       Y.x_blocks = (int)((NH_ + spec_[0].lpw - 1) / spec_[0].lpw);
+      Y.swz = 2 * spec_[0].lpw * (int)sizeof(T) < 128;
       Y.axis = 1;
       Y.Ny = (int)N_[1];
       Y.Nz = nd_ > 2 ? (int)N_[2] : 1;   // stacked firings: no octant index along the firing axis
@@ -1065,6 +1073,7 @@ class Sim final : public SimBase {
       Z.Sa = NHP_ * N_[1];
       Z.So = NHP_;
       Z.x_blocks = (int)((NH_ + spec_[1].lpw - 1) / spec_[1].lpw);
+      Z.swz = 2 * spec_[1].lpw * (int)sizeof(T) < 128;
       Z.axis = 2;
       Z.Ny = (int)N_[1];
       Z.Nz = (int)N_[2];
@@ -1210,11 +1219,11 @@ class Sim final : public SimBase {
   // pass launches on axis a: the compiled-length kernels or their chirp-z form
   hipError_t ldir(int a, const PassCfg& c, const PassArgs<T>& A) {
     return bs_[a] ? launch_dir_bs<T>(c.n, a == 0, c.grid, c.block, c.shmem, stream_, A)
-                  : launch_dir<T>(c.n, a == 0, c.grid, c.block, c.shmem, stream_, A, c.pv);
+                  : launch_dir<T>(c.n, a == 0, c.grid, c.block, c.shmem, stream_, A, c.family());
   }
   hipError_t lspec(int a, const PassCfg& c, const SpecArgs<T>& A) {
     return bs_[a] ? launch_spec_bs<T>(c.n, c.grid, c.block, c.shmem, stream_, A)
-                  : launch_spec<T>(c.n, c.grid, c.block, c.shmem, stream_, A, c.pv);
+                  : launch_spec<T>(c.n, c.grid, c.block, c.shmem, stream_, A, c.family());
   }
   hipError_t lc2r(const PassCfg& c, const C2RArgs<T>& A) {
     return bs_[0] ? launch_c2r_bs<T>(c.n, c.grid, c.block, c.shmem, stream_, A)
@@ -1225,9 +1234,9 @@ class Sim final : public SimBase {
   PassCfg line_cfg(long long n, long long lines, long long outer) {
     PassCfg c;
     c.n = (int)n;
-    const int tpl = plan_tpl((int)n);
+    const int tpl = plan_tpl((int)n, default_family<T>(kStrided));
     const size_t line_bytes = (size_t)plan_pitch((int)n) * sizeof(Cx<T>);
-    int lpw = 256 / tpl;
+    int lpw = std::max(1, 256 / tpl);
     while (lpw > 1 && (size_t)lpw * line_bytes > lds_max_) lpw /= 2;
     while (lpw > 1 && lpw / 2 >= lines) lpw /= 2;
     c.lpw = lpw;
@@ -1392,6 +1401,7 @@ class Sim final : public SimBase {
   bool axisym_ = false;
   DevBuf inv_r_;
   size_t lds_max_ = 65536;   // LDS a workgroup may allocate on this device
+  bool large_ = false;       // the fields exceed the last-level cache
   long long fill_wgs_ = 512;  // workgroups that fill the device (two per CU)
   double c_ref_ = 0, tau_ = 0, y_ = 0, anp_ = 0, d_[3] = {1, 1, 1};
   std::vector<long long> psrc_idx_h_;
@@ -2293,8 +2303,8 @@ int32_t kw_tune_import(const char* text) {
     while (k < 6 && ls >> v[k]) ++k;
     if (!(ls >> std::ws).eof() || (k != 4 && k != 5)) raise(KW_ERR_INVALID, "malformed tuning text");
     const long long p = v[0], c = v[1], n = v[2], l = v[3];
-    if ((p != 4 && p != 8) || c < 0 || c >= TC_COUNT || n < 1 || n > (1 << 20) || !size_supported((int)n) || l < 1 ||
-        l > 256)
+    if ((p != 4 && p != 8) || c < 0 || c >= TC_COUNT || n < 1 || n > (1 << 20) ||
+        !(size_supported((int)n) || direct_size((int)n)) || l < 1 || l > 256)
       raise(KW_ERR_INVALID, "malformed tuning entry");
     if (k == 5 && !plan_alternative((int)n, (int)std::max(-1LL, std::min(v[4], 1000LL))))
       raise(KW_ERR_INVALID, "plan family " + std::to_string(v[4]) + " is not compiled for line length " +

@@ -262,7 +262,7 @@ class ElasticSim {
   }
 
   PassCfg line_cfg(long long n, bool contig, long long lines, long long outer) {
-    return line_pass_cfg(n, contig, lines, outer, sizeof(Cx<T>), lds_max_, fill_wgs_);
+    return line_pass_cfg<T>(n, contig, lines, outer, lds_max_, fill_wgs_);
   }
 
   ElArgs<T> base_args(int axis) {
@@ -273,6 +273,7 @@ class ElasticSim {
     A.Ny = (int)N_[1];
     A.n_lines = (int)(N_[1] * N_[2]);
     A.x_blocks = (int)(((N_[0] + 1) / 2 + c.lpw - 1) / c.lpw);
+    A.swz = swizzled_rows(c.lpw, sizeof(T), N_[0] * (long long)sizeof(T));
     if (axis == 0) {
       A.Sa = 1;
       A.So = N_[0];

@@ -32,6 +32,7 @@ struct ElArgs {
   int Nx;
   long long Sa, So;
   int n_lines, x_blocks;
+  int swz;             // strided: consecutive tiles on one XCD (xcd_wg)
   int Ny;              // grid extent along y (per-line coordinates)
   int axis;            // axis the lines run along
   int ndim;
@@ -97,8 +98,8 @@ __device__ __forceinline__ Cx<T> el_med(const LineCtx<T, N, V>& L, const T* m, T
 // otherwise cost the derivative and normal-stress passes occupancy).
 template <typename T, int N, bool CONTIG, int MODE>
 __global__ void __launch_bounds__(512) k_el_pass(ElArgs<T> a) {
-  constexpr int V = CONTIG ? 2 : 0;  // contiguous lines: plan family 2 (fewer, longer rows per thread)
-  constexpr bool OPQ = dir_opaque<T, N, CONTIG>();   // as for the acoustic directional passes
+  constexpr int V = default_family<T>(CONTIG ? kC2R : kStrided);
+  constexpr bool OPQ = dir_opaque<T, N, CONTIG, V>();   // as for the acoustic directional passes
   constexpr int E = Plan<N, V>::E;
   constexpr int P = LdsLayout<N>::PITCH;
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -111,7 +112,7 @@ __global__ void __launch_bounds__(512) k_el_pass(ElArgs<T> a) {
   geo.x_blocks = a.x_blocks;
   int lpw;
   const LineCtx<T, N, V> L =
-      make_ctx<T, N, CONTIG, V>(geo, CONTIG ? (int)blockIdx.x : strided_wg<T, N>(blockIdx.x), lpw);
+      make_ctx<T, N, CONTIG, V>(geo, CONTIG ? (int)blockIdx.x : strided_wg(blockIdx.x, a.swz), lpw);
   Cx<T>* lds = lds_all + L.c * P;
   const Twiddles<T, N, V> tw = load_twiddles<T, N, V>(a.tw, L.t);
 

@@ -229,126 +229,275 @@ struct DFT<T, 5, INV> {
 template <int... Rs>
 struct Radices {};
 
-// V = 0: plans of the strided and spectral passes (lines spread across
-// workgroup lanes, so more lines per workgroup = wider coalesced rows);
-// V = 1: plans of the contiguous x-line passes, which may trade a larger
-// TPL (fewer registers, more waves) for extra LDS exchanges; V = 2 (below)
-// for the complex-to-real x pass.
+// A plan is a thread count per line and a radix list.  Families (V), each the
+// default of one kind of pass in one precision (default_family):
+//   0 / 3  strided and spectral passes in FP32 / FP64,
+//   1 / 6  contiguous directional x passes in FP32 / FP64,
+//   2 / 7  complex-to-real x pass, the adjoint's r2c stage, contiguous elastic
+//          and operator passes in FP32 / FP64,
+//   4      complex-to-real chirp-z lines in FP32,
+//   8      wide rows: strided and spectral passes in FP32 on grids larger than
+//          the last-level cache (kWideFamily below),
+//   5      lines of the fused y-inverse / complex-to-real plane kernel.
+// What bounds the passes is memory, reached with enough waves in flight: the
+// directional passes carry three to five arrays of E elements per thread, so
+// E <= 8 (FP64) ... 10 keeps them at or below 128 VGPRs (four waves per SIMD)
+// and FP64 out of scratch.  With 16 elements the FP64 128-point x pass spilled
+// 796 bytes per lane and took 85 us on 128^3 (now 31), its strided pass 42
+// (20); with 8 threads per line (32-byte pieces of a row per load) the FP32
+// 128-point x pass took 25 us (now 17).  Lengths with several primes take an
+// uneven pass (StockhamPass) rather than more elements: 240 = 5 x 8 x 6 on 48
+// threads.  Both columns of the table were taken from timed sweeps of radix
+// lists and thread counts at 8 M (FP32) and 4 M (FP64) voxels.
 template <int N, int V = 0>
 struct Plan;
-#define KW_PLAN(N_, TPL_, ...)                     \
+#define KW_PLAN(V_, N_, TPL_, ...)                 \
   template <>                                      \
-  struct Plan<N_, 0> {                             \
+  struct Plan<N_, V_> {                            \
     static constexpr int N = N_;                   \
     static constexpr int TPL = TPL_;               \
     static constexpr int E = N_ / TPL_;            \
     using R = Radices<__VA_ARGS__>;                \
   };
-KW_PLAN(8, 1, 8)
-KW_PLAN(10, 1, 10)
-KW_PLAN(12, 1, 12)
-KW_PLAN(16, 1, 16)
-KW_PLAN(20, 2, 10, 2)
-KW_PLAN(24, 2, 12, 2)
-KW_PLAN(32, 4, 8, 4)
-KW_PLAN(40, 2, 20, 2)
-KW_PLAN(48, 4, 12, 4)
-KW_PLAN(64, 8, 8, 8)
-KW_PLAN(80, 4, 20, 4)
-KW_PLAN(96, 4, 24, 4)
-KW_PLAN(128, 8, 16, 8)
-KW_PLAN(160, 8, 20, 4, 2)
-KW_PLAN(192, 8, 24, 8)
-KW_PLAN(256, 16, 16, 16)
-KW_PLAN(320, 16, 20, 4, 4)
-KW_PLAN(384, 32, 12, 4, 4, 2)
-KW_PLAN(512, 32, 16, 8, 4)
-KW_PLAN(640, 32, 20, 4, 4, 2)
-KW_PLAN(768, 64, 12, 4, 4, 4)
-KW_PLAN(1024, 64, 16, 16, 4)
-KW_PLAN(2048, 128, 16, 16, 8)
-KW_PLAN(4096, 256, 16, 16, 16)
-// odd and other composite lengths (grids need not be powers of two)
-KW_PLAN(9, 1, 9)
-KW_PLAN(15, 1, 15)
-KW_PLAN(25, 5, 5, 5)
-KW_PLAN(27, 3, 9, 3)
-KW_PLAN(36, 3, 12, 3)
-KW_PLAN(45, 3, 15, 3)
-KW_PLAN(72, 6, 12, 6)
-KW_PLAN(75, 5, 15, 5)
-KW_PLAN(81, 9, 9, 9)
-KW_PLAN(100, 10, 10, 10)
-KW_PLAN(125, 25, 5, 5, 5)
-KW_PLAN(135, 9, 15, 3, 3)
-KW_PLAN(144, 12, 12, 12)
-KW_PLAN(200, 10, 20, 10)
-KW_PLAN(225, 15, 15, 15)
-KW_PLAN(243, 27, 9, 9, 3)
-KW_PLAN(400, 20, 20, 20)
-#undef KW_PLAN
+// inherited families (specialised below where another plan is faster)
 template <int N>
 struct Plan<N, 1> : Plan<N, 0> {};
-template <>
-struct Plan<512, 1> {
-  static constexpr int N = 512;
-  static constexpr int TPL = 64;
-  static constexpr int E = 8;
-  using R = Radices<8, 8, 8>;
-};
-template <>
-struct Plan<256, 1> {
-  static constexpr int N = 256;
-  static constexpr int TPL = 64;
-  static constexpr int E = 4;
-  using R = Radices<4, 4, 4, 4>;
-};
-// V = 2: the complex-to-real pass along x (and the adjoint's r2c stage),
-// which carry fewer live arrays than the directional x pass and run faster
-// with more elements per thread.
 template <int N>
-struct Plan<N, 2> : Plan<N, 1> {};
-template <>
-struct Plan<256, 2> {
-  static constexpr int N = 256;
-  static constexpr int TPL = 32;
-  static constexpr int E = 8;
-  using R = Radices<8, 8, 4>;
-};
-
-// V = 5: the lines of the fused y-inverse / complex-to-real plane kernel: the
-// plans of family 2, with twiddles read from the table (the kernel's
-// registers hold a whole plane of the spectrum).
+struct Plan<N, 2> : Plan<N, 0> {};
 template <int N>
-struct Plan<N, 5> : Plan<N, 2> {};
-
-// V = 4: contiguous-line passes (x pass, complex-to-real) of chirp-z lines,
-// which carry the chirp and filter arrays on top of the field arrays: the long
-// plans use 8 elements per thread (the 16-element plans spill registers there).
+struct Plan<N, 3> : Plan<N, 0> {};
 template <int N>
 struct Plan<N, 4> : Plan<N, 1> {};
-template <>
-struct Plan<1024, 4> {
-  static constexpr int N = 1024;
-  static constexpr int TPL = 128;
-  static constexpr int E = 8;
-  using R = Radices<8, 8, 4, 4>;
-};
-template <>
-struct Plan<2048, 4> {
-  static constexpr int N = 2048;
-  static constexpr int TPL = 256;
-  static constexpr int E = 8;
-  using R = Radices<8, 8, 8, 4>;
-};
+template <int N>
+struct Plan<N, 5> : Plan<N, 2> {};
+template <int N>
+struct Plan<N, 6> : Plan<N, 1> {};
+template <int N>
+struct Plan<N, 7> : Plan<N, 3> {};
+template <int N>
+struct Plan<N, 8> : Plan<N, 0> {};
+
+// strided and spectral passes
+KW_PLAN(0, 8, 1, 8)
+KW_PLAN(0, 9, 1, 9)
+KW_PLAN(0, 10, 1, 10)
+KW_PLAN(0, 12, 1, 12)
+KW_PLAN(0, 15, 1, 15)
+KW_PLAN(0, 16, 1, 16)
+KW_PLAN(0, 20, 2, 10, 2)
+KW_PLAN(0, 24, 2, 12, 2)
+KW_PLAN(0, 25, 5, 5, 5)
+KW_PLAN(0, 27, 3, 9, 3)
+KW_PLAN(0, 32, 4, 8, 4)
+KW_PLAN(0, 36, 3, 12, 3)
+KW_PLAN(0, 40, 8, 5, 8)
+KW_PLAN(0, 45, 9, 5, 9)
+KW_PLAN(0, 48, 4, 12, 4)
+KW_PLAN(0, 60, 12, 5, 12)
+KW_PLAN(0, 64, 16, 4, 4, 4)
+KW_PLAN(0, 72, 6, 12, 6)
+KW_PLAN(0, 75, 15, 5, 15)
+KW_PLAN(0, 80, 20, 4, 5, 4)
+KW_PLAN(0, 81, 9, 9, 9)
+KW_PLAN(0, 90, 18, 5, 6, 3)
+KW_PLAN(0, 96, 24, 4, 6, 4)
+KW_PLAN(0, 100, 10, 10, 10)
+KW_PLAN(0, 108, 18, 6, 6, 3)
+KW_PLAN(0, 120, 24, 5, 6, 4)
+KW_PLAN(0, 125, 25, 5, 5, 5)
+KW_PLAN(0, 128, 16, 8, 8, 2)
+KW_PLAN(0, 135, 27, 5, 9, 3)
+KW_PLAN(0, 144, 12, 12, 12)
+KW_PLAN(0, 150, 30, 5, 6, 5)
+KW_PLAN(0, 160, 20, 8, 5, 4)
+KW_PLAN(0, 162, 27, 6, 9, 3)
+KW_PLAN(0, 180, 30, 6, 6, 5)
+KW_PLAN(0, 192, 24, 8, 6, 4)
+KW_PLAN(0, 200, 40, 5, 8, 5)
+KW_PLAN(0, 216, 36, 6, 6, 6)
+KW_PLAN(0, 225, 45, 5, 9, 5)
+KW_PLAN(0, 240, 48, 5, 8, 6)
+KW_PLAN(0, 243, 27, 9, 9, 3)
+KW_PLAN(0, 250, 50, 5, 10, 5)
+KW_PLAN(0, 256, 32, 8, 8, 4)
+KW_PLAN(0, 270, 45, 6, 9, 5)
+KW_PLAN(0, 288, 48, 6, 8, 6)
+KW_PLAN(0, 300, 60, 5, 10, 6)
+KW_PLAN(0, 320, 64, 5, 8, 8)
+KW_PLAN(0, 324, 54, 6, 9, 6)
+KW_PLAN(0, 360, 60, 6, 10, 6)
+KW_PLAN(0, 375, 25, 15, 5, 5)
+KW_PLAN(0, 384, 64, 6, 8, 8)
+KW_PLAN(0, 400, 50, 8, 10, 5)
+KW_PLAN(0, 432, 54, 8, 9, 6)
+KW_PLAN(0, 450, 50, 9, 10, 5)
+KW_PLAN(0, 480, 60, 8, 10, 6)
+KW_PLAN(0, 486, 54, 9, 9, 6)
+KW_PLAN(0, 500, 50, 10, 10, 5)
+KW_PLAN(0, 512, 64, 8, 8, 8)
+KW_PLAN(0, 540, 60, 9, 10, 6)
+KW_PLAN(0, 576, 48, 12, 12, 4)
+KW_PLAN(0, 600, 60, 10, 10, 6)
+KW_PLAN(0, 640, 80, 8, 10, 8)
+KW_PLAN(0, 648, 54, 12, 9, 6)
+KW_PLAN(0, 720, 60, 12, 10, 6)
+KW_PLAN(0, 750, 50, 15, 10, 5)
+KW_PLAN(0, 768, 64, 12, 4, 4, 4)
+KW_PLAN(0, 800, 100, 8, 10, 10)
+KW_PLAN(0, 864, 108, 8, 12, 9)
+KW_PLAN(0, 900, 100, 9, 10, 10)
+KW_PLAN(0, 960, 64, 15, 8, 8)
+KW_PLAN(0, 972, 108, 9, 12, 9)
+KW_PLAN(0, 1000, 100, 10, 10, 10)
+KW_PLAN(0, 1024, 64, 16, 8, 8)
+KW_PLAN(0, 2048, 128, 16, 16, 8)
+KW_PLAN(0, 4096, 256, 16, 16, 16)
+// contiguous directional passes (FP32)
+KW_PLAN(1, 16, 4, 4, 4)
+KW_PLAN(1, 20, 5, 4, 5)
+KW_PLAN(1, 24, 6, 4, 6)
+KW_PLAN(1, 32, 8, 4, 8)
+KW_PLAN(1, 36, 6, 6, 6)
+KW_PLAN(1, 48, 8, 6, 8)
+KW_PLAN(1, 72, 12, 6, 12)
+KW_PLAN(1, 90, 15, 6, 15)
+KW_PLAN(1, 100, 20, 5, 5, 4)
+KW_PLAN(1, 108, 12, 9, 12)
+KW_PLAN(1, 120, 30, 4, 6, 5)
+KW_PLAN(1, 128, 32, 4, 4, 4, 2)
+KW_PLAN(1, 144, 24, 6, 6, 4)
+KW_PLAN(1, 160, 32, 5, 8, 4)
+KW_PLAN(1, 192, 32, 6, 8, 4)
+KW_PLAN(1, 256, 64, 4, 4, 4, 4)
+KW_PLAN(1, 270, 30, 9, 6, 5)
+KW_PLAN(1, 500, 125, 4, 5, 5, 5)
+KW_PLAN(1, 576, 72, 8, 9, 8)
+KW_PLAN(1, 648, 81, 8, 9, 9)
+KW_PLAN(1, 720, 90, 8, 10, 9)
+KW_PLAN(1, 750, 75, 10, 15, 5)
+KW_PLAN(1, 768, 96, 8, 12, 8)
+KW_PLAN(1, 960, 120, 8, 12, 10)
+KW_PLAN(1, 1024, 256, 4, 4, 4, 4, 4)
+KW_PLAN(1, 2048, 256, 8, 8, 8, 4)
+KW_PLAN(1, 4096, 512, 8, 8, 8, 8)
+// wide rows
+KW_PLAN(8, 256, 16, 16, 16)
+KW_PLAN(8, 512, 32, 16, 8, 4)
+KW_PLAN(8, 1024, 64, 16, 16, 4)
+// strided and spectral passes (FP64)
+KW_PLAN(3, 12, 4, 3, 4)
+KW_PLAN(3, 15, 5, 3, 5)
+KW_PLAN(3, 16, 4, 4, 4)
+KW_PLAN(3, 20, 5, 4, 5)
+KW_PLAN(3, 24, 6, 4, 6)
+KW_PLAN(3, 32, 8, 4, 8)
+KW_PLAN(3, 36, 6, 6, 6)
+KW_PLAN(3, 48, 8, 6, 8)
+KW_PLAN(3, 72, 12, 6, 12)
+KW_PLAN(3, 108, 18, 6, 6, 3)
+KW_PLAN(3, 128, 32, 4, 4, 4, 2)
+KW_PLAN(3, 160, 32, 5, 8, 4)
+KW_PLAN(3, 256, 64, 4, 4, 4, 4)
+KW_PLAN(3, 270, 30, 9, 6, 5)
+KW_PLAN(3, 300, 30, 10, 6, 5)
+KW_PLAN(3, 360, 30, 12, 6, 5)
+KW_PLAN(3, 375, 25, 15, 5, 5)
+KW_PLAN(3, 384, 32, 12, 8, 4)
+KW_PLAN(3, 432, 36, 12, 6, 6)
+KW_PLAN(3, 640, 64, 10, 8, 8)
+KW_PLAN(3, 720, 80, 9, 10, 8)
+KW_PLAN(3, 750, 75, 10, 15, 5)
+KW_PLAN(3, 768, 96, 8, 12, 8)
+KW_PLAN(3, 960, 96, 10, 12, 8)
+KW_PLAN(3, 1024, 128, 8, 8, 8, 2)
+KW_PLAN(3, 2048, 256, 8, 8, 8, 4)
+KW_PLAN(3, 4096, 512, 8, 8, 8, 8)
+// contiguous directional passes (FP64)
+KW_PLAN(6, 100, 25, 4, 5, 5)
+KW_PLAN(6, 108, 27, 4, 9, 3)
+KW_PLAN(6, 200, 50, 4, 10, 5)
+KW_PLAN(6, 216, 54, 4, 9, 6)
+KW_PLAN(6, 240, 30, 8, 6, 5)
+KW_PLAN(6, 300, 30, 10, 6, 5)
+KW_PLAN(6, 375, 75, 5, 15, 5)
+KW_PLAN(6, 512, 128, 4, 4, 4, 4, 2)
+KW_PLAN(6, 540, 90, 6, 10, 9)
+KW_PLAN(6, 576, 64, 9, 8, 8)
+KW_PLAN(6, 600, 100, 6, 10, 10)
+KW_PLAN(6, 640, 64, 10, 8, 8)
+KW_PLAN(6, 648, 108, 6, 12, 9)
+KW_PLAN(6, 750, 125, 6, 5, 5, 5)
+// complex-to-real (FP64): at most 256 threads
+KW_PLAN(7, 4096, 256, 16, 16, 16)
+// complex-to-real chirp-z lines, which carry the chirp and filter arrays too
+
+KW_PLAN(4, 1024, 128, 8, 8, 4, 4)
+KW_PLAN(4, 2048, 256, 8, 8, 8, 4)
+KW_PLAN(4, 4096, 256, 16, 16, 16)
+#undef KW_PLAN
+
+enum PassKind { kStrided, kContig, kC2R };
+template <typename T>
+constexpr int default_family(PassKind k, bool chirp = false) {
+  if (sizeof(T) == 8) return k == kStrided ? 3 : (k == kContig ? 6 : 7);
+  return k == kStrided ? 0 : (k == kContig ? 1 : (chirp ? 4 : 2));
+}
+
+// Line pairs per workgroup of a strided pass: the largest power of two that
+// keeps the workgroup at 256 threads, but rows of at least 32 bytes where 512
+// threads allow it.  Workgroups of at most 256 threads leave several of them
+// on a CU, so one computes while others wait for memory or for a barrier; the
+// narrow rows this gives long lines cost no bandwidth as long as neighbouring
+// tiles share an L2 (xcd_wg).  Measured at 8 M FP32 voxels, strided pass: 192
+// points 38 us with 8 pairs (52 with 16), 320 points 48 us with 4 (57 with 8),
+// 256 points 38 us with 8 (41 us with 16 x 16 plans and 16 pairs).
+//
+// Grids larger than the last-level cache (large) stream every field from HBM,
+// where wider rows count more than a fuller CU: rows of 128 bytes where 512
+// threads allow them (512 x 512 x 256 FP32 with FP16 maps, 512-point y pass:
+// 426 us with 4 pairs, 406 with 8; 256-point z pass 429 with 8, 389 with 16,
+// 370 on the 16 x 16 plan of kWideFamily).  Not for lines that do not fill
+// whole waves, which lose more to the barriers of larger workgroups (150-point
+// z pass of 240 x 216 x 150: 53 us with 8 pairs, 62 with 16).
+constexpr int strided_lines(int tpl, int elem_bytes, bool large = false) {
+  int l = 1;
+  while (2 * l * tpl <= 256) l *= 2;
+  while (2 * l * elem_bytes < 32 && 2 * l * tpl <= 512) l *= 2;
+  if (large && 64 % tpl == 0)
+    while (2 * l * elem_bytes < 128 && 2 * l * tpl <= 512) l *= 2;
+  return l;
+}
+// A grid whose `fields` arrays of n elements do not fit the last-level cache.
+constexpr bool beyond_cache(int fields, long long n, int elem_bytes) {
+  return (long long)fields * n * elem_bytes > (256LL << 20);
+}
+// On such grids the FP32 256-point strided passes and the 256-, 512- and
+// 1024-point spectral passes take 16 elements per thread, which gives 128-byte
+// rows to workgroups of 256 or 512 threads: 512 x 512 x 256, spectral y / z
+// passes 125 / 145 us with 8 elements and 110 / 133 with 16; 256^3 35.6 / 37.5
+// and 32.9 / 35.1.  The 512-point directional pass keeps 8 (406 us; 433).
+constexpr int kWideFamily = 8;
+constexpr bool wide_strided(int n) { return n == 256; }
+constexpr bool wide_spectral(int n) { return n == 256 || n == 512 || n == 1024; }
+// Lines per workgroup of a contiguous pass: 256 threads where several lines
+// share a wave, one line where it fills waves of its own (256^3 x pass: 120 us
+// with 1, 123 with 4; 512 x 512 x 256: 490 and 506), else about 192 threads
+// (240 points on 48 threads, 8 M FP32 voxels: 68 us with 4 pairs, 92 with 8).
+constexpr int contig_lines(int tpl) {
+  const int th = 64 % tpl == 0 ? (tpl == 64 ? 64 : 256) : (tpl % 64 == 0 ? tpl : 192);
+  return th / tpl > 0 ? th / tpl : 1;
+}
 
 // LDS slice of one line: one complex of padding per 16 keeps the
-// stride-16/32 Stockham writes off a single bank group.  The 4096 plan is
-// left unpadded so a double-precision line still fits a 64 KiB workgroup.
+// stride-16/32 Stockham writes off a single bank group, and an odd pitch keeps
+// the lines of a strided pass, whose lanes run across them, on different banks
+// (240 + 15 + 1 = 256 put all of them on one: strided pass 97 us instead of
+// 58).  The 4096 plan is left unpadded so a double-precision line still fits a
+// 64 KiB workgroup.
 template <int N>
 struct LdsLayout {
   static constexpr bool PAD = N >= 16 && N < 4096;
-  static constexpr int PITCH = PAD ? N + N / 16 + 1 : N;
+  static constexpr int PITCH = PAD ? (N + N / 16) | 1 : N;
   __device__ __forceinline__ static int at(int i) { return PAD ? i + (i >> 4) : i; }
 };
 
@@ -365,15 +514,19 @@ struct RadixArray {
 template <int... Rs>
 constexpr int RadixArray<Rs...>::r[];
 
+// Butterflies of radix r that a thread of a line of n points on tpl threads
+// computes: the line's n / r butterflies are dealt to the threads in turn.
+constexpr int butterflies_per_thread(int n, int tpl, int r) { return (n / r + tpl - 1) / tpl; }
+
 template <int N, int V, typename RL>
 struct TwCount;
 template <int N, int V, int... Rs>
 struct TwCount<N, V, Radices<Rs...>> {
   static constexpr int f() {
     constexpr int rr[] = {Rs...};
-    int E = N / Plan<N, V>::TPL, Ns = 1, tot = 0;
+    int Ns = 1, tot = 0;
     for (int i = 0; i < (int)sizeof...(Rs); ++i) {
-      if (Ns > 1) tot += (E / rr[i]) * (rr[i] - 1);
+      if (Ns > 1) tot += butterflies_per_thread(N, Plan<N, V>::TPL, rr[i]) * (rr[i] - 1);
       Ns *= rr[i];
     }
     return tot;
@@ -392,11 +545,11 @@ struct Twiddles {
 template <typename T, int N, int V, int TPL, int Ns, int OFF, int R, int... Rest>
 struct TwLoad {
   __device__ __forceinline__ static void run(Twiddles<T, N, V>& tw, const Cx<T>* __restrict__ table, int t) {
-    constexpr int NB = (N / TPL) / R;
+    constexpr int NB = butterflies_per_thread(N, TPL, R);
     if constexpr (Ns > 1) {
 #pragma unroll
       for (int m = 0; m < NB; ++m) {
-        const int jm = (t + TPL * m) % Ns;
+        const int jm = (t + TPL * m) % Ns;   // in the table also for a butterfly that no thread computes
 #pragma unroll
         for (int r = 1; r < R; ++r) tw.w[OFF + m * (R - 1) + (r - 1)] = table[jm * r * (N / (Ns * R))];
       }
@@ -453,12 +606,22 @@ struct StockhamNext<T, N, V, TPL, INV, Ns, OFF, WAVE> {
 template <typename T, int N, int V, int TPL, bool INV, int Ns, int OFF, bool WAVE, int R, int... Rest>
 struct StockhamPass {
   static constexpr int E = N / TPL;
-  static constexpr int NB = E / R;
-  static_assert(E % R == 0, "radix must divide the per-thread element count");
+  // A radix that divides E keeps the stride-TPL layout: butterfly j of thread
+  // t = j % TPL finds its inputs in the thread's registers.  Any other radix
+  // (an uneven pass, never the first) takes its inputs from the exchange
+  // instead, its butterflies dealt to the threads in turn, the last round not
+  // full: lengths such as 240 = 15 x 16 then need 15 elements per thread and
+  // two exchanges, where a radix list that divides E would need 30 or 60.
+  static constexpr bool EVEN = E % R == 0;
+  static constexpr int NB = butterflies_per_thread(N, TPL, R);
+  static constexpr bool FULL = (N / R) % TPL == 0;   // every thread has NB butterflies
+  static_assert(EVEN || Ns > 1, "the first radix must divide the per-thread element count");
   // this pass reads its twiddles from the table (plans too large to keep
   // them in registers); NW of them per thread
   static constexpr bool TAB = !Twiddles<T, N, V>::REG && Ns > 1;
   static constexpr int NW = TAB ? NB * (R - 1) : 1;
+  static constexpr bool LAST = sizeof...(Rest) == 0;
+  static_assert(!LAST || Ns * R == N, "radix product must equal N");
   using Next =
       typename StockhamNext<T, N, V, TPL, INV, Ns * R, (Ns > 1 ? OFF + NB * (R - 1) : OFF), WAVE, Rest...>::type;
 
@@ -477,36 +640,67 @@ struct StockhamPass {
     fetch(w, tw, t);
     body(v, lds, tw, t, w);
   }
-  // w: this pass's table twiddles, fetched by the caller
+  // w: this pass's table twiddles, fetched by the caller.  EVEN: v holds the
+  // line in the stride-TPL layout; else the line is in LDS, in order.
   __device__ __forceinline__ static void body(Cx<T> (&v)[E], Cx<T>* lds, const Twiddles<T, N, V>& tw, int t,
                                               const Cx<T> (&w)[NW]) {
-    constexpr bool LAST = sizeof...(Rest) == 0;
-    static_assert(!LAST || Ns * R == N, "radix product must equal N");
+    if constexpr (EVEN) {
 #pragma unroll
-    for (int m = 0; m < NB; ++m) {
-      Cx<T> x[R];
+      for (int m = 0; m < NB; ++m) {
+        Cx<T> x[R];
 #pragma unroll
-      for (int r = 0; r < R; ++r) x[r] = v[m + r * NB];
-      const int j = t + TPL * m;
-      if constexpr (Ns > 1) {
+        for (int r = 0; r < R; ++r) x[r] = v[m + r * NB];
+        const int j = t + TPL * m;
+        if constexpr (Ns > 1) {
 #pragma unroll
-        for (int r = 1; r < R; ++r) {
-          Cx<T> wr;
-          if constexpr (Twiddles<T, N, V>::REG)
-            wr = tw.w[OFF + m * (R - 1) + (r - 1)];
-          else
-            wr = w[m * (R - 1) + (r - 1)];
-          x[r] = INV ? cmulc(x[r], wr) : cmul(x[r], wr);
+          for (int r = 1; r < R; ++r) {
+            Cx<T> wr;
+            if constexpr (Twiddles<T, N, V>::REG)
+              wr = tw.w[OFF + m * (R - 1) + (r - 1)];
+            else
+              wr = w[m * (R - 1) + (r - 1)];
+            x[r] = INV ? cmulc(x[r], wr) : cmul(x[r], wr);
+          }
+        }
+        DFT<T, R, INV>::run(x);
+        if constexpr (LAST) {
+#pragma unroll
+          for (int r = 0; r < R; ++r) v[m + r * NB] = x[r];
+        } else {
+          const int base = (j / Ns) * Ns * R + (j % Ns);
+#pragma unroll
+          for (int r = 0; r < R; ++r) lds[LdsLayout<N>::at(base + r * Ns)] = x[r];
         }
       }
-      DFT<T, R, INV>::run(x);
-      if constexpr (LAST) {
+    } else {
+      Cx<T> x[NB][R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) v[m + r * NB] = x[r];
-      } else {
-        const int base = (j / Ns) * Ns * R + (j % Ns);
+      for (int m = 0; m < NB; ++m) {
+        const int j = t + TPL * m;
+        if (FULL || j < N / R) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) lds[LdsLayout<N>::at(base + r * Ns)] = x[r];
+          for (int r = 0; r < R; ++r) x[m][r] = lds[LdsLayout<N>::at(j + r * (N / R))];
+        }
+      }
+      lds_sync<WAVE>();   // every input is read before the outputs replace it
+#pragma unroll
+      for (int m = 0; m < NB; ++m) {
+        const int j = t + TPL * m;
+        if (FULL || j < N / R) {
+#pragma unroll
+          for (int r = 1; r < R; ++r) {
+            Cx<T> wr;
+            if constexpr (Twiddles<T, N, V>::REG)
+              wr = tw.w[OFF + m * (R - 1) + (r - 1)];
+            else
+              wr = w[m * (R - 1) + (r - 1)];
+            x[m][r] = INV ? cmulc(x[m][r], wr) : cmul(x[m][r], wr);
+          }
+          DFT<T, R, INV>::run(x[m]);
+          const int base = (j / Ns) * Ns * R + (j % Ns);
+#pragma unroll
+          for (int r = 0; r < R; ++r) lds[LdsLayout<N>::at(base + r * Ns)] = x[m][r];
+        }
       }
     }
     if constexpr (!LAST) {
@@ -515,10 +709,17 @@ struct StockhamPass {
       Cx<T> wn[Next::NW];
       Next::fetch(wn, tw, t);
       lds_sync<WAVE>();
+      if constexpr (Next::EVEN) {
+#pragma unroll
+        for (int q = 0; q < E; ++q) v[q] = lds[LdsLayout<N>::at(t + TPL * q)];
+        lds_sync<WAVE>();
+      }
+      Next::body(v, lds, tw, t, wn);
+    } else if constexpr (!EVEN) {
+      lds_sync<WAVE>();
 #pragma unroll
       for (int q = 0; q < E; ++q) v[q] = lds[LdsLayout<N>::at(t + TPL * q)];
       lds_sync<WAVE>();
-      Next::body(v, lds, tw, t, wn);
     }
   }
 };

@@ -128,7 +128,7 @@ std::vector<T> to_t(const std::vector<double>& v) {
   return o;
 }
 
-// Chirp-z (Bluestein) tables of a line of length n on the power-of-two plan m
+// Chirp-z (Bluestein) tables of a line of length n on the plan of m points
 // (kw_fft.hpp line_dft), FP64: c_j = exp(-i pi (j^2 mod 2n) / n) for j < n;
 // gf = FFT_m(g) / m with g_k = conj(c_k) for 0 <= k < n and g_(m-k) = conj(c_k)
 // for 0 < k < n (zero elsewhere); gb the same for the filter of c (inverse
@@ -162,6 +162,31 @@ inline void host_fft_pow2(std::vector<double>& re, std::vector<double>& im) {
       }
   }
 }
+// Forward DFT of length m = r 2^a with r odd: the r interleaved power-of-two
+// subsequences F_s, then X_k = sum_s exp(-2 pi i s k / m) F_s[k mod m/r].
+inline void host_fft(std::vector<double>& re, std::vector<double>& im) {
+  const size_t m = re.size();
+  size_t p = 1;
+  while (m % (2 * p) == 0) p *= 2;
+  const size_t r = m / p;
+  std::vector<double> xr(m, 0.0), xi(m, 0.0);
+  for (size_t s = 0; s < r; ++s) {
+    std::vector<double> fr(p), fi(p);
+    for (size_t j = 0; j < p; ++j) {
+      fr[j] = re[r * j + s];
+      fi[j] = im[r * j + s];
+    }
+    host_fft_pow2(fr, fi);
+    for (size_t k = 0; k < m; ++k) {
+      const double a = -2.0 * M_PI * (double)(s * k % m) / (double)m;
+      const double wr = std::cos(a), wi = std::sin(a);
+      xr[k] += fr[k % p] * wr - fi[k % p] * wi;
+      xi[k] += fr[k % p] * wi + fi[k % p] * wr;
+    }
+  }
+  re.swap(xr);
+  im.swap(xi);
+}
 inline ChirpTables chirp_tables(long long n, long long m) {
   ChirpTables C;
   C.cr.resize(n);
@@ -183,7 +208,7 @@ inline ChirpTables chirp_tables(long long n, long long m) {
         gi[m - k] = sg * C.ci[k];
       }
     }
-    host_fft_pow2(gr, gi);
+    host_fft(gr, gi);
     for (long long k = 0; k < m; ++k) {
       gr[k] /= (double)m;
       gi[k] /= (double)m;
@@ -240,9 +265,18 @@ struct PassCfg {
   int lpw = 1;      // lines (pairs) per workgroup
   int req = 1;      // lines per workgroup asked for (before shrinking to small grids)
   int pv = -1;      // plan family (plan_alternative) or -1 for the pass's default
+  bool wide = false;   // the default is the wide-row family (kWideFamily) on this grid
+  int family() const { return wide ? kw::kWideFamily : pv; }   // as the launchers take it
   dim3 grid, block;
   size_t shmem = 0;
 };
+
+// Fewest lines per workgroup a pass on a small grid is split to: one wave, and
+// for strided passes rows of 32 bytes.
+inline int min_lines(bool contig, int tpl, int elem_bytes) {
+  const int wave = std::max(1, 64 / tpl);
+  return contig ? wave : std::max(wave, 32 / (2 * elem_bytes));
+}
 
 // Lines per workgroup of a line pass: 256 threads on contiguous lines, >= 16
 // line pairs up to 512 threads on strided lines, halved until the lines fit
@@ -250,18 +284,21 @@ struct PassCfg {
 // operator tests) use plan family 2 on contiguous lines.
 // fill_wgs > 0: on small grids, fewer lines per workgroup until the launch has
 // fill_wgs workgroups (keeping one full wave per workgroup).
-inline PassCfg line_pass_cfg(long long n, bool contig, long long lines, long long outer, size_t cx_bytes,
-                             size_t lds_max, long long fill_wgs = 0) {
+template <typename T>
+PassCfg line_pass_cfg(long long n, bool contig, long long lines, long long outer, size_t lds_max,
+                      long long fill_wgs = 0) {
   PassCfg c;
   c.n = (int)n;
-  const int tpl = kw::plan_tpl((int)n, contig ? 2 : 0);
-  const size_t line_bytes = (size_t)kw::plan_pitch((int)n) * cx_bytes;
-  int lpw = (contig ? 256 : std::max(256, std::min(512, 16 * tpl))) / tpl;
-  while (lpw > 1 && (size_t)lpw * line_bytes > lds_max) lpw /= 2;
+  const int tpl = kw::plan_tpl((int)n, kw::default_family<T>(contig ? kw::kC2R : kw::kStrided));
+  const size_t line_bytes = (size_t)kw::plan_pitch((int)n) * sizeof(kw::Cx<T>);
   const long long pairs = (lines + 1) / 2;
+  // the elastic solver's nine fields, two partial sums and three maps
+  const bool large = !contig && kw::beyond_cache(14, n * lines * std::max<long long>(outer, 1), sizeof(T));
+  int lpw = contig ? kw::contig_lines(tpl) : kw::strided_lines(tpl, sizeof(T), large);
+  while (lpw > 1 && (size_t)lpw * line_bytes > lds_max) lpw /= 2;
   while (lpw > 1 && lpw / 2 >= pairs) lpw /= 2;
   {
-    const int min_lpw = std::max(1, 64 / tpl);
+    const int min_lpw = min_lines(contig, tpl, sizeof(T));
     const long long o = contig ? 1 : std::max<long long>(outer, 1);
     while (lpw / 2 >= min_lpw && ((pairs + lpw - 1) / lpw) * o < fill_wgs) lpw /= 2;
   }

@@ -34,21 +34,26 @@ __device__ __forceinline__ int xcd_wg(int b, int n) {
   return x < r ? x * (q + 1) + s : r * (q + 1) + (x - r) * q + s;
 }
 // Strided and spectral passes whose workgroups cover less than 128 bytes of
-// each row even at 512 threads (lines of 768 points and more in FP32: 8 line
-// pairs) use it, so the two workgroups reading the halves of one 128-byte
-// segment run on one XCD and the second read hits its L2.  Wider rows keep
-// the plain order (decided at compile time: a runtime test cost the 256-point
-// passes about 1 %).
+// each row, or rows that do not start on a 128-byte boundary, use it, so the
+// workgroups reading the parts of one 128-byte segment run on one XCD and only
+// the first read misses its L2.  Measured on the FP32 strided pass at 8 M
+// voxels: 192 points with 64-byte rows 60 us in the plain order, 38 in this
+// one; 256 points with 8 pairs on rows of 240 voxels 55 and 38.  Aligned
+// 128-byte rows gain nothing (36 us plain, 38) and keep the plain order.  The
+// host decides per launch (`swz` in the arguments, swizzled_rows); batched
+// launches, which mix grids, by the default lines per workgroup of the length.
+inline bool swizzled_rows(int lpw, int elem_bytes, long long row_pitch_bytes) {
+  return 2 * lpw * elem_bytes < 128 || row_pitch_bytes % 128 != 0;
+}
+__device__ __forceinline__ int strided_wg(unsigned b, int swz) {
+  return swz ? xcd_wg((int)b, (int)gridDim.x) : (int)b;
+}
 template <typename T, int N>
-__device__ __forceinline__ int strided_wg(int b, int n) {
-  if constexpr ((512 / Plan<N, 0>::TPL) * 2 * (int)sizeof(T) < 128)
+__device__ __forceinline__ int strided_wg_batch(int b, int n) {
+  if constexpr (strided_lines(Plan<N, default_family<T>(kStrided)>::TPL, sizeof(T)) * 2 * (int)sizeof(T) < 128)
     return xcd_wg(b, n);
   else
     return b;
-}
-template <typename T, int N>
-__device__ __forceinline__ int strided_wg(int b) {
-  return strided_wg<T, N>(b, (int)gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -90,6 +95,7 @@ struct PassArgs {
   int n_outer;     // outer count
   int n_lines;     // contiguous: number of real lines
   int x_blocks;    // strided: workgroups along x
+  int swz;         // strided: consecutive tiles on one XCD (xcd_wg)
   // sources
   SrcList psrc;
   SrcList usrc;
@@ -322,8 +328,8 @@ struct LineCtx {
   }
 };
 
-// VV selects the plan family (default: 1 for contiguous x lines, 0 for strided).
-template <typename T, int N, bool CONTIG, int VV = (CONTIG ? 1 : 0), bool BS = false>
+// VV selects the plan family.
+template <typename T, int N, bool CONTIG, int VV, bool BS = false>
 __device__ __forceinline__ LineCtx<T, N, VV, BS> make_ctx(const PassArgs<T>& a, int wg, int& lpw_out) {
   constexpr int V = VV;
   constexpr int TPL = Plan<N, V>::TPL;
@@ -403,15 +409,14 @@ __device__ __forceinline__ void inject(const SrcList& s, int t_index, Cx<T> (&v)
 // passes on 16-element plans (128 ... 4096 points) run at two waves per SIMD
 // either way, and there the merged addresses are faster (512-point strided
 // pass of the 512^3 step: 0.94 ms merged, 1.00 ms separate).
-template <typename T, int N, bool CONTIG, int V = (CONTIG ? 1 : 0)>
+template <typename T, int N, bool CONTIG, int V>
 constexpr bool dir_opaque() {
   return CONTIG || Plan<N, V>::E != 16;
 }
 
 // Plan families a pass can be launched with besides its default (the
-// autotuner's choice of radix decomposition and threads per line): at 256
-// points 16 x 16 (family 0), 64 x 4 (1) and 32 x 8 (2); at 512 points 32 x 16
-// (0) and 64 x 8 (1, 2).  PV = -1 in a kernel's template arguments selects the
+// autotuner's choice of radix decomposition and threads per line), at 256 and
+// 512 points: 32 x 8 (family 0), 64 x 4 (1) and 32 x 8 (2); 64 x 8.  PV = -1 in a kernel's template arguments selects the
 // pass's default family.
 constexpr bool plan_alternative(int n, int v) {
   return (n == 256 || n == 512) && v >= 0 && v <= 2;
@@ -419,7 +424,7 @@ constexpr bool plan_alternative(int n, int v) {
 
 template <typename T, int N, bool CONTIG, bool TWO = false, bool BS = false, int PV = -1>
 __device__ __forceinline__ void dir_pass_body(const PassArgs<T>& a, int wg, int t_index) {
-  constexpr int V = PV >= 0 ? PV : (CONTIG ? (BS ? 4 : 1) : 0);   // plan family
+  constexpr int V = PV >= 0 ? PV : default_family<T>(CONTIG ? kContig : kStrided, CONTIG && BS);   // plan family
   constexpr bool WL = CONTIG && wave_local_lines<N, V>();   // lines inside one wavefront
   constexpr bool OPQ = dir_opaque<T, N, CONTIG, V>();
   constexpr int E = Plan<N, V>::E;
@@ -659,7 +664,7 @@ __device__ __forceinline__ void dir_pass_body(const PassArgs<T>& a, int wg, int 
 
 template <typename T, int N, bool CONTIG, bool TWO = false, bool BS = false, int PV = -1>
 __global__ void __launch_bounds__(512) k_dir_pass(PassArgs<T> a) {
-  dir_pass_body<T, N, CONTIG, TWO, BS, PV>(a, CONTIG ? (int)blockIdx.x : strided_wg<T, N>(blockIdx.x), a.t);
+  dir_pass_body<T, N, CONTIG, TWO, BS, PV>(a, CONTIG ? (int)blockIdx.x : strided_wg(blockIdx.x, a.swz), a.t);
 }
 
 // Batched form: one launch covers the nwg workgroup tiles of many
@@ -679,7 +684,7 @@ constexpr bool persistent_length(int n) { return n == 256 || n == 384 || n == 51
 template <typename T, int N, bool CONTIG, bool TWO>
 __device__ __forceinline__ void dir_tile(const PassArgs<T>* __restrict__ args, const int* __restrict__ wg_sim,
                                       const int* __restrict__ wg_first, int t, int w, int nwg) {
-  const int b = CONTIG ? w : strided_wg<T, N>(w, nwg);
+  const int b = CONTIG ? w : strided_wg_batch<T, N>(w, nwg);
   const int s = cmem(wg_sim)[b];
   const PassArgs<T> a = cmem(args)[s];
   dir_pass_body<T, N, CONTIG, TWO>(a, b - cmem(wg_first)[s], t);
@@ -696,7 +701,7 @@ __global__ void __launch_bounds__(512) k_dir_pass_batch(const PassArgs<T>* __res
       dir_tile<T, N, CONTIG, TWO>(args, wg_sim, wg_first, t, w, nwg);
     }
   } else {
-    const int b = CONTIG ? (int)blockIdx.x : strided_wg<T, N>(blockIdx.x);
+    const int b = CONTIG ? (int)blockIdx.x : strided_wg_batch<T, N>(blockIdx.x, (int)gridDim.x);
     const int s = cmem(wg_sim)[b];
     const PassArgs<T> a = cmem(args)[s];
     dir_pass_body<T, N, CONTIG, TWO>(a, b - cmem(wg_first)[s], *cmem(t_dev));
@@ -718,6 +723,7 @@ struct SpecArgs {
   long long Sa;       // stride along the line (complex elements)
   long long So;       // outer stride
   int x_blocks;
+  int swz;            // consecutive tiles on one XCD (xcd_wg)
   int mode;           // 0 fwd, 1 inv, 2 fwd*M*inv, 3 fwd*W*inv (1-D window W along the line)
   const T* W;         // mode 3 window (length N, 1/N folded in)
   // octant table addressing: index = kx + MH1*(|line index| + MH2*|outer index|)
@@ -735,7 +741,7 @@ struct SpecArgs {
 // keeps the plain transforms at a small register footprint.
 template <typename T, int N, int MODE, bool BS = false, int PV = -1>
 __device__ __forceinline__ void spec_pass_body(const SpecArgs<T>& a, int wg) {
-  constexpr int V = PV >= 0 ? PV : 0;   // plan family
+  constexpr int V = PV >= 0 ? PV : default_family<T>(kStrided);   // plan family
   constexpr int TPL = Plan<N, V>::TPL;
   constexpr int E = Plan<N, V>::E;
   constexpr int P = LdsLayout<N>::PITCH;
@@ -862,13 +868,13 @@ __device__ __forceinline__ void spec_pass_body(const SpecArgs<T>& a, int wg) {
 
 template <typename T, int N, int MODE, bool BS = false, int PV = -1>
 __global__ void __launch_bounds__(512) k_spec_pass(SpecArgs<T> a) {
-  spec_pass_body<T, N, MODE, BS, PV>(a, strided_wg<T, N>(blockIdx.x));
+  spec_pass_body<T, N, MODE, BS, PV>(a, strided_wg(blockIdx.x, a.swz));
 }
 
 template <typename T, int N, int MODE>
 __device__ __forceinline__ void spec_tile(const SpecArgs<T>* __restrict__ args, const int* __restrict__ wg_sim,
                                        const int* __restrict__ wg_first, int w, int nwg) {
-  const int b = strided_wg<T, N>(w, nwg);
+  const int b = strided_wg_batch<T, N>(w, nwg);
   const int s = cmem(wg_sim)[b];
   const SpecArgs<T> a = cmem(args)[s];
   spec_pass_body<T, N, MODE>(a, b - cmem(wg_first)[s]);
@@ -884,7 +890,7 @@ __global__ void __launch_bounds__(512) k_spec_pass_batch(const SpecArgs<T>* __re
       spec_tile<T, N, MODE>(args, wg_sim, wg_first, w, nwg);
     }
   } else {
-    const int b = strided_wg<T, N>(blockIdx.x);
+    const int b = strided_wg_batch<T, N>(blockIdx.x, (int)gridDim.x);
     const int s = cmem(wg_sim)[b];
     const SpecArgs<T> a = cmem(args)[s];
     spec_pass_body<T, N, MODE>(a, b - cmem(wg_first)[s]);
@@ -912,8 +918,8 @@ struct C2RArgs {
 
 template <typename T, int N, bool BS = false, int PV = -1>
 __device__ __forceinline__ void c2r_body(const C2RArgs<T>& a, int wg) {
-  // contiguous x lines, complex-to-real plan family (4: chirp-z lines)
-  constexpr int V = PV >= 0 ? PV : (BS ? 4 : 2);
+  // contiguous x lines
+  constexpr int V = PV >= 0 ? PV : default_family<T>(kC2R, BS);
   constexpr int TPL = Plan<N, V>::TPL;
   constexpr int E = Plan<N, V>::E;
   constexpr int P = LdsLayout<N>::PITCH;
@@ -1403,12 +1409,13 @@ struct AdjArgs {
   int Nx;
   long long Sa, So;
   int n_lines, x_blocks;
+  int swz;          // strided: consecutive tiles on one XCD (xcd_wg)
   int accumulate;   // 0: Pb = contribution, 1: Pb += contribution
 };
 
 template <typename T, int N, bool CONTIG, int PV = -1>
 __global__ void __launch_bounds__(512) k_adj_pass(AdjArgs<T> a) {
-  constexpr int V = PV >= 0 ? PV : (CONTIG ? 1 : 0);   // plan family, as the directional pass's
+  constexpr int V = PV >= 0 ? PV : default_family<T>(CONTIG ? kContig : kStrided);   // as the directional pass's
   constexpr bool OPQ = dir_opaque<T, N, CONTIG, V>();
   constexpr int E = Plan<N, V>::E;
   constexpr int P = LdsLayout<N>::PITCH;
@@ -1422,7 +1429,7 @@ __global__ void __launch_bounds__(512) k_adj_pass(AdjArgs<T> a) {
   geo.x_blocks = a.x_blocks;
   int lpw;
   const LineCtx<T, N, V> L =
-      make_ctx<T, N, CONTIG, V>(geo, CONTIG ? (int)blockIdx.x : strided_wg<T, N>(blockIdx.x), lpw);
+      make_ctx<T, N, CONTIG, V>(geo, CONTIG ? (int)blockIdx.x : strided_wg(blockIdx.x, a.swz), lpw);
   Cx<T>* lds = lds_all + L.c * P;
   const Twiddles<T, N, V> tw = load_twiddles<T, N, V>(a.tw, L.t);
 
@@ -1496,7 +1503,7 @@ __global__ void __launch_bounds__(512) k_adj_pass(AdjArgs<T> a) {
 // Real lines (pairs) of f -> half spectrum along x (the r2c stage alone).
 template <typename T, int N, int PV = -1>
 __global__ void __launch_bounds__(256) k_r2c_x(const T* f, Cx<T>* S, int n_lines, int nhp, const Cx<T>* twt) {
-  constexpr int V = PV >= 0 ? PV : 2;  // contiguous x lines: the complex-to-real pass's plan family
+  constexpr int V = PV >= 0 ? PV : default_family<T>(kC2R);  // contiguous x lines
   constexpr int E = Plan<N, V>::E;
   constexpr int P = LdsLayout<N>::PITCH;
   constexpr int NH = N / 2 + 1;

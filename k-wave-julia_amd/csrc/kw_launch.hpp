@@ -12,28 +12,44 @@
   X(80) X(81) X(96) X(100) X(125) X(128) X(135) X(144) X(160) X(192) X(200) X(225) X(243) X(256) X(320)  \
   X(384) X(400) X(512) X(640) X(768) X(1024) X(2048) X(4096)
 
-// Power-of-two plans that carry lines of any other length (Bluestein).
-#define KW_BS_SIZES(X) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024) X(2048) X(4096)
+// Further products of 2, 3 and 5 with a plan of their own.  Single simulations
+// run them directly; batches, the adjoint, the elastic solver and the operator
+// entry points do not take them (size_supported), as for any other length
+// outside KW_SIZES.
+#define KW_DIRECT_SIZES(X) \
+  X(60) X(90) X(108) X(120) X(150) X(162) X(180) X(216) X(240) X(250) X(270) X(288) X(300) X(324) X(360) X(375) \
+  X(432) X(450) X(480) X(486) X(500) X(540) X(576) X(600) X(648) X(720) X(750) X(800) X(864) X(900) X(960)      \
+  X(972) X(1000)
+
+// Plans that carry lines of any other length (Bluestein): powers of two, and
+// 3 and 5 times a power of two between them, so that a line of length n runs
+// on at most 4/3 (2n - 1) points (n = 300: 640 points instead of 1024).
+#define KW_BS_SIZES(X) \
+  X(8) X(16) X(32) X(64) X(96) X(128) X(192) X(256) X(320) X(384) X(512) X(640) X(768) X(1024) X(2048) X(4096)
 
 namespace kw {
 
 bool size_supported(long long n);
-// Plan length of a line of length n without a compiled plan: the power of two
-// n_plan >= 2n - 1 (at least 8) on which its chirp-z transform runs; 0 if n is
-// longer than the largest plan allows (n > 2048).
+// Lengths in KW_DIRECT_SIZES.
+bool direct_size(long long n);
+// Plan length of a line of length n without a compiled plan: the smallest
+// n_plan >= 2n - 1 in KW_BS_SIZES, on which its chirp-z transform runs; 0 if n
+// is longer than the largest plan allows (n > 2048).
 inline long long bluestein_plan(long long n) {
   if (n < 1) return 0;
-  long long m = 8;
-  while (m < 2 * n - 1) m <<= 1;
-  return m <= 4096 ? m : 0;
+#define X(m_) \
+  if (m_ >= 2 * n - 1) return m_;
+  KW_BS_SIZES(X)
+#undef X
+  return 0;
 }
 // grid of the adjoint's reduction kernels (one partial-sum slot per block)
 inline unsigned adj_reduce_blocks(long long n) {
   const long long nb = (n + 255) / 256;
   return nb < 1 ? 1u : (nb < 1024 ? (unsigned)nb : 1024u);
 }
-// variant 1: contiguous x-line passes, 2: complex-to-real x pass, 4: both for chirp-z lines
-int plan_tpl(int n, int variant = 0);
+// threads per line of length n in plan family `family` (0 where n has no plan)
+int plan_tpl(int n, int family);
 int plan_pitch(int n);
 
 // Return hipSuccess or the launch error; unsupported lengths give hipErrorInvalidValue.

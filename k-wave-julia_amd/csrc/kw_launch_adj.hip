@@ -35,6 +35,11 @@ static hipError_t r2c_alt(int pv, dim3 g, dim3 b, size_t sh, hipStream_t s, cons
 template <typename T>
 hipError_t launch_adj_pass(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const AdjArgs<T>& a,
                            int pv) {
+  if constexpr (sizeof(T) == 4)
+    if (pv == kWideFamily && !contig && n == 256) {
+      hipLaunchKernelGGL((k_adj_pass<T, 256, false, kWideFamily>), g, b, sh, s, a);
+      return hipGetLastError();
+    }
   if (plan_alternative(n, pv))
     return n == 256 ? adj_alt<T, 256>(pv, contig, g, b, sh, s, a) : adj_alt<T, 512>(pv, contig, g, b, sh, s, a);
   switch (n) {

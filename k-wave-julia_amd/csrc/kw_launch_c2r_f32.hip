@@ -23,6 +23,7 @@ hipError_t launch_c2r<float>(int n, dim3 g, dim3 b, size_t sh, hipStream_t s, co
     hipLaunchKernelGGL((k_c2r_x<float, n_>), g, b, sh, s, a);        \
     return hipGetLastError();
     KW_SIZES(X)
+    KW_DIRECT_SIZES(X)
 #undef X
   }
   return hipErrorInvalidValue;

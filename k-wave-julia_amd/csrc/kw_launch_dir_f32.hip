@@ -27,6 +27,10 @@ static hipError_t dir_alt(int pv, bool contig, dim3 g, dim3 b, size_t sh, hipStr
 template <>
 hipError_t launch_dir<float>(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const PassArgs<float>& a,
                            int pv) {
+  if (pv == kWideFamily && !contig && n == 256) {
+    hipLaunchKernelGGL((k_dir_pass<float, 256, false, false, false, kWideFamily>), g, b, sh, s, a);
+    return hipGetLastError();
+  }
   if (plan_alternative(n, pv)) return n == 256 ? dir_alt<256>(pv, contig, g, b, sh, s, a) : dir_alt<512>(pv, contig, g, b, sh, s, a);
   switch (n) {
 #define X(n_)                                                                  \
@@ -39,6 +43,7 @@ hipError_t launch_dir<float>(int n, bool contig, dim3 g, dim3 b, size_t sh, hipS
       hipLaunchKernelGGL((k_dir_pass<float, n_, false>), g, b, sh, s, a);       \
     return hipGetLastError();
     KW_SIZES(X)
+    KW_DIRECT_SIZES(X)
 #undef X
   }
   return hipErrorInvalidValue;

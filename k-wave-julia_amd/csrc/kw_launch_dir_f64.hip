@@ -39,6 +39,7 @@ hipError_t launch_dir<double>(int n, bool contig, dim3 g, dim3 b, size_t sh, hip
       hipLaunchKernelGGL((k_dir_pass<double, n_, false>), g, b, sh, s, a);       \
     return hipGetLastError();
     KW_SIZES(X)
+    KW_DIRECT_SIZES(X)
 #undef X
   }
   return hipErrorInvalidValue;

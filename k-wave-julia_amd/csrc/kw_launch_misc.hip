@@ -40,13 +40,28 @@ bool size_supported(long long n) {
   }
 }
 
-int plan_tpl(int n, int variant) {
+bool direct_size(long long n) {
   switch (n) {
-#define X(n_) \
-  case n_:    \
-    return variant == 4 ? Plan<n_, 4>::TPL                                                  \
-                        : (variant == 2 ? Plan<n_, 2>::TPL : (variant ? Plan<n_, 1>::TPL : Plan<n_, 0>::TPL));
+#define X(n_) case n_:
+    KW_DIRECT_SIZES(X)
+#undef X
+    return true;
+    default:
+      return false;
+  }
+}
+
+int plan_tpl(int n, int family) {
+  switch (n) {
+#define X(n_)                                                                                                        \
+  case n_: {                                                                                                         \
+    static constexpr int tpl[9] = {Plan<n_, 0>::TPL, Plan<n_, 1>::TPL, Plan<n_, 2>::TPL, Plan<n_, 3>::TPL,            \
+                                   Plan<n_, 4>::TPL, Plan<n_, 5>::TPL, Plan<n_, 6>::TPL, Plan<n_, 7>::TPL,            \
+                                   Plan<n_, 8>::TPL};                                                                \
+    return family >= 0 && family < 9 ? tpl[family] : 0;                                                              \
+  }
     KW_SIZES(X)
+    KW_DIRECT_SIZES(X)
 #undef X
   }
   return 0;
@@ -58,6 +73,7 @@ int plan_pitch(int n) {
   case n_:    \
     return LdsLayout<n_>::PITCH;
     KW_SIZES(X)
+    KW_DIRECT_SIZES(X)
 #undef X
   }
   return 0;

@@ -75,12 +75,18 @@ static hipError_t spec_alt(int pv, dim3 g, dim3 b, size_t sh, hipStream_t s, con
 
 template <>
 hipError_t launch_spec<float>(int n, dim3 g, dim3 b, size_t sh, hipStream_t s, const SpecArgs<float>& a, int pv) {
+  if (pv == kWideFamily) switch (n) {
+      case 256: return spec_alt<256, kWideFamily>(g, b, sh, s, a);
+      case 512: return spec_alt<512, kWideFamily>(g, b, sh, s, a);
+      case 1024: return spec_alt<1024, kWideFamily>(g, b, sh, s, a);
+    }
   if (plan_alternative(n, pv)) return n == 256 ? spec_alt<256>(pv, g, b, sh, s, a) : spec_alt<512>(pv, g, b, sh, s, a);
   switch (n) {
 #define X(n_)   \
   case n_:      \
     return spec_mode<n_, float>(a.mode, g, b, sh, s, a);
     KW_SIZES(X)
+    KW_DIRECT_SIZES(X)
 #undef X
   }
   return hipErrorInvalidValue;

@@ -81,6 +81,7 @@ hipError_t launch_spec<double>(int n, dim3 g, dim3 b, size_t sh, hipStream_t s, 
   case n_:      \
     return spec_mode<n_, double>(a.mode, g, b, sh, s, a);
     KW_SIZES(X)
+    KW_DIRECT_SIZES(X)
 #undef X
   }
   return hipErrorInvalidValue;

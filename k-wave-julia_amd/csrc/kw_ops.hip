@@ -85,6 +85,7 @@ ElArgs<T> deriv_args(const long long n[3], int ndim, int axis, const PassCfg& c,
   a.Ny = (int)n[1];
   a.n_lines = (int)(n[1] * n[2]);
   a.x_blocks = (int)(((n[0] + 1) / 2 + c.lpw - 1) / c.lpw);
+  a.swz = swizzled_rows(c.lpw, sizeof(T), n[0] * (long long)sizeof(T));
   a.Sa = axis == 0 ? 1 : (axis == 1 ? n[0] : n[0] * n[1]);
   a.So = axis == 0 ? n[0] : (axis == 1 ? n[0] * n[1] : n[0]);
   a.axis = axis;
@@ -101,7 +102,7 @@ PassCfg deriv_cfg(int dev, const long long n[3], int axis) {
   HIPC(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
   const long long L = n[axis], lines = n[0] * n[1] * n[2] / L;
   const long long outer = axis == 0 ? 0 : (axis == 1 ? n[2] : n[1]);
-  return line_pass_cfg(L, axis == 0, axis == 0 ? lines : n[0], outer, sizeof(Cx<T>), lds > 0 ? (size_t)lds : 65536);
+  return line_pass_cfg<T>(L, axis == 0, axis == 0 ? lines : n[0], outer, lds > 0 ? (size_t)lds : 65536);
 }
 
 // Argument checks shared by both derivative entry points.
