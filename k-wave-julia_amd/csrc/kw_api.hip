@@ -16,6 +16,7 @@
 #include "../../include/kwave_hip.h"
 #include "kw_host.hpp"
 #include "kw_launch.hpp"
+#include "kw_line1d.hpp"
 
 using namespace kw;
 using namespace kwh;
@@ -105,7 +106,11 @@ class Sim final : public SimBase {
 
   void run(long long n) override {
     HIPC(hipSetDevice(dev_));
-    for (long long i = 0; i < n && t_ < Nt_; ++i) step(nullptr);
+    if (line1d_) {
+      run_line1d(std::min(n, Nt_ - t_));
+    } else {
+      for (long long i = 0; i < n && t_ < Nt_; ++i) step(nullptr);
+    }
     HIPC(hipGetLastError());
     if (t_ == Nt_ && !finalized_) finalize();
   }
@@ -1092,6 +1097,9 @@ class Sim final : public SimBase {
     ca_.n_lines = (int)(N_[1] * N_[2]);
     // the fused y-inverse / c2r plane pass where the plane fits a workgroup
     plane_c2r_ = nd_ == 3 && !batch_mode_ && !bs_[0] && !bs_[1] && plane_c2r_supported<T>((int)N_[0], (int)N_[1], lds_max_);
+    // a 1-D grid whose line and recorder buffers fit a workgroup's LDS
+    const size_t l1 = nd_ == 1 && !batch_mode_ ? line1d_lds_bytes<T>((int)M_[0], bs_[0]) : 0;
+    line1d_ = l1 > 0 && l1 <= lds_max_;
     std::memset(&plane_args_, 0, sizeof(plane_args_));
     plane_args_.S1 = S1_.as<Cx<T>>();
     plane_args_.tw_x = tw_[0].as<Cx<T>>();
@@ -1246,6 +1254,31 @@ class Sim final : public SimBase {
     return c;
   }
 
+  // ---- 1-D grids: many steps per launch, in one workgroup -------------------
+  void run_line1d(long long n) {
+    Line1dArgs<T> a;
+    std::memset(&a, 0, sizeof(a));
+    a.x = pa_[0];
+    a.p = p_.as<T>();
+    a.M1 = M1_.as<T>();
+    a.M2 = stokes_ ? M2_.as<T>() : nullptr;
+    a.rec = ra_;
+    if (!(nsens_ > 0 && !cartesian_ && rec_)) a.rec.n = 0;
+    if (tr_ && tr_vals_.p && nsens_ > 0) {
+      a.tr_idx = sidx_tr();
+      a.tr_vals = tr_vals_.as<T>();
+      a.tr_n = (int)nsens_;
+    }
+    a.Nt = (int)Nt_;
+    while (n > 0) {
+      a.nsteps = (int)std::min<long long>(n, 256);   // about a millisecond per launch
+      a.t0 = (int)t_ + 1;
+      HIPC(launch_line1d<T>((int)M_[0], bs_[0], stream_, a));
+      t_ += a.nsteps;
+      n -= a.nsteps;
+    }
+  }
+
   // ---- one time step ------------------------------------------------------
   void step(Prof* pr) {
     const int t = (int)(++t_);
@@ -1368,6 +1401,7 @@ class Sim final : public SimBase {
   bool bs_[3] = {false, false, false};   // axis runs chirp-z (Bluestein) lines
   DevBuf chc_[3], chf_[3], chb_[3];       // chirp tables of those axes
   int nfire_ = 1;          // stacked firings (2-D), 1 otherwise
+  bool line1d_ = false;    // 1-D: run() steps in one workgroup (k_line1d)
   bool plane_c2r_ = false; // 3-D step: y inverse and c2r fused per z plane
   PlaneArgs<T> plane_args_{};
   long long plane_ = 0;    // voxels of one firing's grid

@@ -757,7 +757,7 @@ constexpr bool wave_local_lines() {
 template <typename T, int N, bool INV, int V = 0, bool WAVE = false, bool OPQ = false>
 __device__ __forceinline__ void line_fft(Cx<T> (&v)[(Plan<N, V>::E)], Cx<T>* lds, const Twiddles<T, N, V>& tw,
                                          int t) {
-  static_assert(!WAVE || 64 % Plan<N, V>::TPL == 0, "wave-local lines need TPL dividing 64");
+  static_assert(!WAVE || Plan<N, V>::TPL <= 64, "wave-local lines have at most 64 threads");
   LineFFTImpl<T, N, V, INV, WAVE, OPQ, typename Plan<N, V>::R>::run(v, lds, tw, t);
 }
 

@@ -1168,26 +1168,26 @@ struct RecArgs {
   double* I_max;
 };
 
+// Whether a record selection needs the velocities.
+constexpr bool records_u(unsigned rec) {
+  return (rec & (REC_UX | REC_UY | REC_UZ | REC_U_MAX | REC_U_RMS | REC_U_FINAL | REC_I_AVG | REC_I_MAX)) != 0;
+}
+// Sensor row j takes pressure pv and velocities uv (ndim of them) of step t_index.
 template <typename T>
-__device__ __forceinline__ void record_body(const RecArgs<T>& a, int j, int t_index) {
-  const long long i = a.idx ? a.idx[j] : (long long)j;   // null: every voxel, in order
-  const T pv = a.p[i];
+__device__ __forceinline__ void record_values(const RecArgs<T>& a, int j, int t_index, T pv, const T (&uv)[3],
+                                              int ndim) {
   const long long o = (long long)(t_index - 1) * a.n + j;
   if (a.rec & REC_P) a.p_ts[o] = pv;
   if (a.rec & REC_P_MAX) a.p_max[j] = a.p_max[j] > pv ? a.p_max[j] : pv;
   if (a.rec & REC_P_MIN) a.p_min[j] = a.p_min[j] < pv ? a.p_min[j] : pv;
   if (a.rec & REC_P_RMS) a.p_rms[j] += (double)pv * (double)pv;
   if ((a.rec & REC_P_FINAL) && t_index == a.Nt) a.p_final[j] = pv;
-  T uv[3] = {0, 0, 0};
-  // velocities only when a velocity or intensity field is recorded
-  if (a.rec & (REC_UX | REC_UY | REC_UZ | REC_U_MAX | REC_U_RMS | REC_U_FINAL | REC_I_AVG | REC_I_MAX))
-    for (int d = 0; d < a.ndim; ++d) uv[d] = a.u[d][i];
   if (a.rec & REC_UX) a.u_ts[0][o] = uv[0];
-  if ((a.rec & REC_UY) && a.ndim > 1) a.u_ts[1][o] = uv[1];
-  if ((a.rec & REC_UZ) && a.ndim > 2) a.u_ts[2][o] = uv[2];
+  if ((a.rec & REC_UY) && ndim > 1) a.u_ts[1][o] = uv[1];
+  if ((a.rec & REC_UZ) && ndim > 2) a.u_ts[2][o] = uv[2];
   if (a.rec & (REC_U_MAX | REC_U_RMS | REC_U_FINAL)) {
     double m2 = 0.0;
-    for (int d = 0; d < a.ndim; ++d) m2 += (double)uv[d] * (double)uv[d];
+    for (int d = 0; d < ndim; ++d) m2 += (double)uv[d] * (double)uv[d];
     const double mag = sqrt(m2);
     if (a.rec & REC_U_MAX) a.u_max[j] = a.u_max[j] > mag ? a.u_max[j] : mag;
     if (a.rec & REC_U_RMS) a.u_rms[j] += mag * mag;
@@ -1195,7 +1195,7 @@ __device__ __forceinline__ void record_body(const RecArgs<T>& a, int j, int t_in
   }
   if (a.rec & (REC_I_AVG | REC_I_MAX)) {
     double s = 0.0;
-    for (int d = 0; d < a.ndim; ++d) {
+    for (int d = 0; d < ndim; ++d) {
       const double pu = (double)pv * (double)uv[d];
       s += pu * pu;
     }
@@ -1203,6 +1203,15 @@ __device__ __forceinline__ void record_body(const RecArgs<T>& a, int j, int t_in
     if (a.rec & REC_I_AVG) a.I_avg[j] += inst / a.Nt;
     if (a.rec & REC_I_MAX) a.I_max[j] = a.I_max[j] > inst ? a.I_max[j] : inst;
   }
+}
+
+template <typename T>
+__device__ __forceinline__ void record_body(const RecArgs<T>& a, int j, int t_index) {
+  const long long i = a.idx ? a.idx[j] : (long long)j;   // null: every voxel, in order
+  T uv[3] = {0, 0, 0};
+  if (records_u(a.rec))
+    for (int d = 0; d < a.ndim; ++d) uv[d] = a.u[d][i];
+  record_values<T>(a, j, t_index, a.p[i], uv, a.ndim);
 }
 
 template <typename T>
