@@ -383,13 +383,33 @@ __device__ __forceinline__ void inject(const SrcList& s, int t_index, Cx<T> (&v)
   __syncthreads();
   const int col = (t_index < s.ncols ? t_index : s.ncols) - 1;
   const T* vals = reinterpret_cast<const T*>(s.val) + (long long)col * s.n_src;
-  for (int e = e0 + (int)threadIdx.x; e < e1; e += blockDim.x) {
-    const int pk = s.pos[e];
-    const int n = pk & 0xFFFFF, part = (pk >> 20) & 1, c = pk >> 21;
-    const T val = vals[s.row[e]];
-    Cx<T>& cell = lds_all[c * P + LdsLayout<N>::at(n)];
-    T& dst = part ? cell.y : cell.x;
-    dst = s.dirichlet ? val : dst + val;
+  // Entries in groups of B per thread, so that their position, row and value
+  // loads overlap: a plane source puts thousands of entries on the few
+  // workgroups of its plane, and one entry at a time each waits for three
+  // dependent loads (128^3 FP32 with a source plane: y pass 23.6 us, 18.3 in
+  // groups of 4, which cost no registers; groups of 8 took the x pass from 78
+  // to 91).
+  constexpr int B = 4;
+  const int nt = (int)blockDim.x;
+  for (int eb = e0 + (int)threadIdx.x; eb < e1; eb += B * nt) {
+    int pk[B], rw[B];
+    T val[B];
+#pragma unroll
+    for (int k = 0; k < B; ++k) {
+      const int e = eb + k * nt < e1 ? eb + k * nt : eb;
+      pk[k] = s.pos[e];
+      rw[k] = s.row[e];
+    }
+#pragma unroll
+    for (int k = 0; k < B; ++k) val[k] = vals[rw[k]];
+#pragma unroll
+    for (int k = 0; k < B; ++k) {
+      if (eb + k * nt >= e1) break;
+      const int n = pk[k] & 0xFFFFF, part = (pk[k] >> 20) & 1, c = pk[k] >> 21;
+      Cx<T>& cell = lds_all[c * P + LdsLayout<N>::at(n)];
+      T& dst = part ? cell.y : cell.x;
+      dst = s.dirichlet ? val[k] : dst + val[k];
+    }
   }
   __syncthreads();
 #pragma unroll
