@@ -45,9 +45,10 @@ __device__ __forceinline__ int xcd_wg(int b, int n) {
 inline bool swizzled_rows(int lpw, int elem_bytes, long long row_pitch_bytes) {
   return 2 * lpw * elem_bytes < 128 || row_pitch_bytes % 128 != 0;
 }
-__device__ __forceinline__ int strided_wg(unsigned b, int swz) {
-  return swz ? xcd_wg((int)b, (int)gridDim.x) : (int)b;
+__device__ __forceinline__ int strided_wg(unsigned b, int swz, unsigned n) {
+  return swz ? xcd_wg((int)b, (int)n) : (int)b;
 }
+__device__ __forceinline__ int strided_wg(unsigned b, int swz) { return strided_wg(b, swz, gridDim.x); }
 template <typename T, int N>
 __device__ __forceinline__ int strided_wg_batch(int b, int n) {
   if constexpr (strided_lines(Plan<N, default_family<T>(kStrided)>::TPL, sizeof(T)) * 2 * (int)sizeof(T) < 128)
@@ -418,6 +419,94 @@ __device__ __forceinline__ void inject(const SrcList& s, int t_index, Cx<T> (&v)
 }
 
 // ---------------------------------------------------------------------------
+// Sensor recording (record_sensor_data!, first_order_steps.jl:728-794)
+// ---------------------------------------------------------------------------
+enum : unsigned {
+  REC_P = 1u << 0,
+  REC_P_MAX = 1u << 1,
+  REC_P_MIN = 1u << 2,
+  REC_P_RMS = 1u << 3,
+  REC_P_FINAL = 1u << 4,
+  REC_UX = 1u << 5,
+  REC_UY = 1u << 6,
+  REC_UZ = 1u << 7,
+  REC_U_MAX = 1u << 8,
+  REC_U_RMS = 1u << 9,
+  REC_U_FINAL = 1u << 10,
+  REC_I_AVG = 1u << 11,
+  REC_I_MAX = 1u << 12,
+};
+
+template <typename T>
+struct RecArgs {
+  const T* p;
+  const T* u[3];
+  int ndim;
+  const long long* idx;  // sensor voxel of each row, or null when the mask is the whole grid
+  int n;
+  int t;       // 1-based
+  int Nt;
+  unsigned rec;
+  T* p_ts;     // [t][j]
+  T* u_ts[3];  // [t][j]
+  T* p_max;
+  T* p_min;
+  double* p_rms;
+  T* p_final;
+  double* u_max;
+  double* u_rms;
+  double* u_final;
+  double* I_avg;
+  double* I_max;
+};
+
+// Whether a record selection needs the velocities.
+constexpr bool records_u(unsigned rec) {
+  return (rec & (REC_UX | REC_UY | REC_UZ | REC_U_MAX | REC_U_RMS | REC_U_FINAL | REC_I_AVG | REC_I_MAX)) != 0;
+}
+// Sensor row j takes pressure pv and velocities uv (ndim of them) of step t_index.
+template <typename T>
+__device__ __forceinline__ void record_values(const RecArgs<T>& a, int j, int t_index, T pv, const T (&uv)[3],
+                                              int ndim) {
+  const long long o = (long long)(t_index - 1) * a.n + j;
+  if (a.rec & REC_P) a.p_ts[o] = pv;
+  if (a.rec & REC_P_MAX) a.p_max[j] = a.p_max[j] > pv ? a.p_max[j] : pv;
+  if (a.rec & REC_P_MIN) a.p_min[j] = a.p_min[j] < pv ? a.p_min[j] : pv;
+  if (a.rec & REC_P_RMS) a.p_rms[j] += (double)pv * (double)pv;
+  if ((a.rec & REC_P_FINAL) && t_index == a.Nt) a.p_final[j] = pv;
+  if (a.rec & REC_UX) a.u_ts[0][o] = uv[0];
+  if ((a.rec & REC_UY) && ndim > 1) a.u_ts[1][o] = uv[1];
+  if ((a.rec & REC_UZ) && ndim > 2) a.u_ts[2][o] = uv[2];
+  if (a.rec & (REC_U_MAX | REC_U_RMS | REC_U_FINAL)) {
+    double m2 = 0.0;
+    for (int d = 0; d < ndim; ++d) m2 += (double)uv[d] * (double)uv[d];
+    const double mag = sqrt(m2);
+    if (a.rec & REC_U_MAX) a.u_max[j] = a.u_max[j] > mag ? a.u_max[j] : mag;
+    if (a.rec & REC_U_RMS) a.u_rms[j] += mag * mag;
+    if ((a.rec & REC_U_FINAL) && t_index == a.Nt) a.u_final[j] = mag;
+  }
+  if (a.rec & (REC_I_AVG | REC_I_MAX)) {
+    double s = 0.0;
+    for (int d = 0; d < ndim; ++d) {
+      const double pu = (double)pv * (double)uv[d];
+      s += pu * pu;
+    }
+    const double inst = sqrt(s);
+    if (a.rec & REC_I_AVG) a.I_avg[j] += inst / a.Nt;
+    if (a.rec & REC_I_MAX) a.I_max[j] = a.I_max[j] > inst ? a.I_max[j] : inst;
+  }
+}
+
+template <typename T>
+__device__ __forceinline__ void record_body(const RecArgs<T>& a, int j, int t_index) {
+  const long long i = a.idx ? a.idx[j] : (long long)j;   // null: every voxel, in order
+  T uv[3] = {0, 0, 0};
+  if (records_u(a.rec))
+    for (int d = 0; d < a.ndim; ++d) uv[d] = a.u[d][i];
+  record_values<T>(a, j, t_index, a.p[i], uv, a.ndim);
+}
+
+// ---------------------------------------------------------------------------
 // Directional pass (contiguous x lines or strided y/z lines)
 // ---------------------------------------------------------------------------
 // TWO (x pass only): the variant that can also form the second spectrum of
@@ -682,9 +771,22 @@ __device__ __forceinline__ void dir_pass_body(const PassArgs<T>& a, int wg, int 
   }
 }
 
+// The strided passes only read p, so the first of a step can carry the sensor
+// gather of the step before: workgroups from `tiles` on record the rows of r
+// (pressure records only; r.t is that step's index).  As a launch of its own
+// the gather costs 2 us of a 34-us step (512^2 FP32) and 3 of 79 (128^3).
 template <typename T, int N, bool CONTIG, bool TWO = false, bool BS = false, int PV = -1>
-__global__ void __launch_bounds__(512) k_dir_pass(PassArgs<T> a) {
-  dir_pass_body<T, N, CONTIG, TWO, BS, PV>(a, CONTIG ? (int)blockIdx.x : strided_wg(blockIdx.x, a.swz), a.t);
+__global__ void __launch_bounds__(512) k_dir_pass(PassArgs<T> a, RecArgs<T> r, unsigned tiles) {
+  if constexpr (CONTIG) {
+    dir_pass_body<T, N, CONTIG, TWO, BS, PV>(a, (int)blockIdx.x, a.t);
+  } else {
+    if (blockIdx.x >= tiles) {
+      const int j = (int)((blockIdx.x - tiles) * blockDim.x + threadIdx.x);
+      if (j < r.n) record_body<T>(r, j, r.t);
+      return;
+    }
+    dir_pass_body<T, N, CONTIG, TWO, BS, PV>(a, strided_wg(blockIdx.x, a.swz, tiles), a.t);
+  }
 }
 
 // Batched form: one launch covers the nwg workgroup tiles of many
@@ -1147,93 +1249,8 @@ __global__ void __launch_bounds__(1024) k_plane_c2r(PlaneArgs<T> a) {
 }
 
 // ---------------------------------------------------------------------------
-// Sensor recording (record_sensor_data!, first_order_steps.jl:728-794)
+// Sensor recording as a pass of its own
 // ---------------------------------------------------------------------------
-enum : unsigned {
-  REC_P = 1u << 0,
-  REC_P_MAX = 1u << 1,
-  REC_P_MIN = 1u << 2,
-  REC_P_RMS = 1u << 3,
-  REC_P_FINAL = 1u << 4,
-  REC_UX = 1u << 5,
-  REC_UY = 1u << 6,
-  REC_UZ = 1u << 7,
-  REC_U_MAX = 1u << 8,
-  REC_U_RMS = 1u << 9,
-  REC_U_FINAL = 1u << 10,
-  REC_I_AVG = 1u << 11,
-  REC_I_MAX = 1u << 12,
-};
-
-template <typename T>
-struct RecArgs {
-  const T* p;
-  const T* u[3];
-  int ndim;
-  const long long* idx;  // sensor voxel of each row, or null when the mask is the whole grid
-  int n;
-  int t;       // 1-based
-  int Nt;
-  unsigned rec;
-  T* p_ts;     // [t][j]
-  T* u_ts[3];  // [t][j]
-  T* p_max;
-  T* p_min;
-  double* p_rms;
-  T* p_final;
-  double* u_max;
-  double* u_rms;
-  double* u_final;
-  double* I_avg;
-  double* I_max;
-};
-
-// Whether a record selection needs the velocities.
-constexpr bool records_u(unsigned rec) {
-  return (rec & (REC_UX | REC_UY | REC_UZ | REC_U_MAX | REC_U_RMS | REC_U_FINAL | REC_I_AVG | REC_I_MAX)) != 0;
-}
-// Sensor row j takes pressure pv and velocities uv (ndim of them) of step t_index.
-template <typename T>
-__device__ __forceinline__ void record_values(const RecArgs<T>& a, int j, int t_index, T pv, const T (&uv)[3],
-                                              int ndim) {
-  const long long o = (long long)(t_index - 1) * a.n + j;
-  if (a.rec & REC_P) a.p_ts[o] = pv;
-  if (a.rec & REC_P_MAX) a.p_max[j] = a.p_max[j] > pv ? a.p_max[j] : pv;
-  if (a.rec & REC_P_MIN) a.p_min[j] = a.p_min[j] < pv ? a.p_min[j] : pv;
-  if (a.rec & REC_P_RMS) a.p_rms[j] += (double)pv * (double)pv;
-  if ((a.rec & REC_P_FINAL) && t_index == a.Nt) a.p_final[j] = pv;
-  if (a.rec & REC_UX) a.u_ts[0][o] = uv[0];
-  if ((a.rec & REC_UY) && ndim > 1) a.u_ts[1][o] = uv[1];
-  if ((a.rec & REC_UZ) && ndim > 2) a.u_ts[2][o] = uv[2];
-  if (a.rec & (REC_U_MAX | REC_U_RMS | REC_U_FINAL)) {
-    double m2 = 0.0;
-    for (int d = 0; d < ndim; ++d) m2 += (double)uv[d] * (double)uv[d];
-    const double mag = sqrt(m2);
-    if (a.rec & REC_U_MAX) a.u_max[j] = a.u_max[j] > mag ? a.u_max[j] : mag;
-    if (a.rec & REC_U_RMS) a.u_rms[j] += mag * mag;
-    if ((a.rec & REC_U_FINAL) && t_index == a.Nt) a.u_final[j] = mag;
-  }
-  if (a.rec & (REC_I_AVG | REC_I_MAX)) {
-    double s = 0.0;
-    for (int d = 0; d < ndim; ++d) {
-      const double pu = (double)pv * (double)uv[d];
-      s += pu * pu;
-    }
-    const double inst = sqrt(s);
-    if (a.rec & REC_I_AVG) a.I_avg[j] += inst / a.Nt;
-    if (a.rec & REC_I_MAX) a.I_max[j] = a.I_max[j] > inst ? a.I_max[j] : inst;
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ void record_body(const RecArgs<T>& a, int j, int t_index) {
-  const long long i = a.idx ? a.idx[j] : (long long)j;   // null: every voxel, in order
-  T uv[3] = {0, 0, 0};
-  if (records_u(a.rec))
-    for (int d = 0; d < a.ndim; ++d) uv[d] = a.u[d][i];
-  record_values<T>(a, j, t_index, a.p[i], uv, a.ndim);
-}
-
 template <typename T>
 __global__ void __launch_bounds__(256) k_record(RecArgs<T> a) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;

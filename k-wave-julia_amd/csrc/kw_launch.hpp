@@ -54,9 +54,10 @@ int plan_pitch(int n);
 
 // Return hipSuccess or the launch error; unsupported lengths give hipErrorInvalidValue.
 template <typename T>
+// rec (strided passes): also records these sensor rows (k_dir_pass).
 // pv: plan family (plan_alternative), -1 for the pass's default.
 hipError_t launch_dir(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const PassArgs<T>& a,
-                      int pv = -1);
+                      int pv = -1, const RecArgs<T>* rec = nullptr);
 template <typename T>
 hipError_t launch_spec(int n, dim3 g, dim3 b, size_t sh, hipStream_t s, const SpecArgs<T>& a, int pv = -1);
 template <typename T>
@@ -70,7 +71,8 @@ template <typename T>
 hipError_t launch_plane_c2r(int nx, int ny, unsigned nz, hipStream_t s, const PlaneArgs<T>& a);
 // Bluestein forms (n_plan from bluestein_plan; the args carry the line length and chirp tables).
 template <typename T>
-hipError_t launch_dir_bs(int n_plan, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const PassArgs<T>& a);
+hipError_t launch_dir_bs(int n_plan, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const PassArgs<T>& a,
+                         const RecArgs<T>* rec = nullptr);
 template <typename T>
 hipError_t launch_spec_bs(int n_plan, dim3 g, dim3 b, size_t sh, hipStream_t s, const SpecArgs<T>& a);
 template <typename T>

@@ -6,16 +6,19 @@ namespace kw {
 
 template <>
 hipError_t launch_dir_bs<double>(int n_plan, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s,
-                               const PassArgs<double>& a) {
+                               const PassArgs<double>& a, const RecArgs<double>* rec) {
+  const unsigned tiles = g.x;
+  const RecArgs<double> r = rec ? *rec : RecArgs<double>{};
+  if (rec && !contig) g.x += ((unsigned)r.n + b.x - 1) / b.x;
   switch (n_plan) {
 #define X(n_)                                                                          \
   case n_:                                                                             \
     if (contig && a.S2)                                                                \
-      hipLaunchKernelGGL((k_dir_pass<double, n_, true, true, true>), g, b, sh, s, a);      \
+      hipLaunchKernelGGL((k_dir_pass<double, n_, true, true, true>), g, b, sh, s, a, r, tiles);      \
     else if (contig)                                                                   \
-      hipLaunchKernelGGL((k_dir_pass<double, n_, true, false, true>), g, b, sh, s, a);     \
+      hipLaunchKernelGGL((k_dir_pass<double, n_, true, false, true>), g, b, sh, s, a, r, tiles);     \
     else                                                                               \
-      hipLaunchKernelGGL((k_dir_pass<double, n_, false, false, true>), g, b, sh, s, a);    \
+      hipLaunchKernelGGL((k_dir_pass<double, n_, false, false, true>), g, b, sh, s, a, r, tiles);    \
     return hipGetLastError();
     KW_BS_SIZES(X)
 #undef X

@@ -5,38 +5,43 @@ namespace kw {
 
 // the 256- and 512-point passes in an alternative plan family
 template <int N, int PV>
-static hipError_t dir_alt(bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const PassArgs<double>& a) {
+static hipError_t dir_alt(bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const PassArgs<double>& a,
+                          const RecArgs<double>& r, unsigned tiles) {
   if (contig && a.S2)
-    hipLaunchKernelGGL((k_dir_pass<double, N, true, true, false, PV>), g, b, sh, s, a);
+    hipLaunchKernelGGL((k_dir_pass<double, N, true, true, false, PV>), g, b, sh, s, a, r, tiles);
   else if (contig)
-    hipLaunchKernelGGL((k_dir_pass<double, N, true, false, false, PV>), g, b, sh, s, a);
+    hipLaunchKernelGGL((k_dir_pass<double, N, true, false, false, PV>), g, b, sh, s, a, r, tiles);
   else
-    hipLaunchKernelGGL((k_dir_pass<double, N, false, false, false, PV>), g, b, sh, s, a);
+    hipLaunchKernelGGL((k_dir_pass<double, N, false, false, false, PV>), g, b, sh, s, a, r, tiles);
   return hipGetLastError();
 }
 template <int N>
-static hipError_t dir_alt(int pv, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const PassArgs<double>& a) {
+static hipError_t dir_alt(int pv, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const PassArgs<double>& a,
+                          const RecArgs<double>& r, unsigned tiles) {
   switch (pv) {
-    case 0: return dir_alt<N, 0>(contig, g, b, sh, s, a);
-    case 1: return dir_alt<N, 1>(contig, g, b, sh, s, a);
-    case 2: return dir_alt<N, 2>(contig, g, b, sh, s, a);
+    case 0: return dir_alt<N, 0>(contig, g, b, sh, s, a, r, tiles);
+    case 1: return dir_alt<N, 1>(contig, g, b, sh, s, a, r, tiles);
+    case 2: return dir_alt<N, 2>(contig, g, b, sh, s, a, r, tiles);
   }
   return hipErrorInvalidValue;
 }
 
 template <>
 hipError_t launch_dir<double>(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const PassArgs<double>& a,
-                           int pv) {
-  if (plan_alternative(n, pv)) return n == 256 ? dir_alt<256>(pv, contig, g, b, sh, s, a) : dir_alt<512>(pv, contig, g, b, sh, s, a);
+                           int pv, const RecArgs<double>* rec) {
+  const unsigned tiles = g.x;
+  const RecArgs<double> r = rec ? *rec : RecArgs<double>{};
+  if (rec && !contig) g.x += ((unsigned)r.n + b.x - 1) / b.x;
+  if (plan_alternative(n, pv)) return n == 256 ? dir_alt<256>(pv, contig, g, b, sh, s, a, r, tiles) : dir_alt<512>(pv, contig, g, b, sh, s, a, r, tiles);
   switch (n) {
 #define X(n_)                                                                  \
   case n_:                                                                     \
     if (contig && a.S2)                                                        \
-      hipLaunchKernelGGL((k_dir_pass<double, n_, true, true>), g, b, sh, s, a);  \
+      hipLaunchKernelGGL((k_dir_pass<double, n_, true, true>), g, b, sh, s, a, r, tiles);  \
     else if (contig)                                                           \
-      hipLaunchKernelGGL((k_dir_pass<double, n_, true, false>), g, b, sh, s, a); \
+      hipLaunchKernelGGL((k_dir_pass<double, n_, true, false>), g, b, sh, s, a, r, tiles); \
     else                                                                       \
-      hipLaunchKernelGGL((k_dir_pass<double, n_, false>), g, b, sh, s, a);       \
+      hipLaunchKernelGGL((k_dir_pass<double, n_, false>), g, b, sh, s, a, r, tiles);       \
     return hipGetLastError();
     KW_SIZES(X)
     KW_DIRECT_SIZES(X)
