@@ -617,6 +617,7 @@ class Sim final : public SimBase {
     plane_ = nvox_ / nfire_;
     // p, u_d, rho_d, two maps and the half spectrum; a batch's launches mix grids
     large_ = !batch_mode_ && beyond_cache(2 * nd_ + 4, nvox_, (int)sizeof(T));
+    rev_ = !batch_mode_ && beyond_cache(nd_ + 2, nvox_, (int)sizeof(T));
     NH_ = N_[0] / 2 + 1;
     NHP_ = (NH_ + 15) / 16 * 16;  // 128-byte aligned spectrum rows (FP32)
     dt_ = d.dt;
@@ -1005,7 +1006,8 @@ class Sim final : public SimBase {
       A.ch = chirp(a);
       const PassCfg& c = cfg_[a];
       A.x_blocks = (int)(((N_[0] + 1) / 2 + c.lpw - 1) / c.lpw);
-      A.swz = a > 0 && swizzled_rows(c.lpw, sizeof(T), N_[0] * (long long)sizeof(T));
+      A.swz = a > 0 ? tile_order(c.lpw, sizeof(T), N_[0] * (long long)sizeof(T), A.x_blocks, large_) : 0;
+      A.rev = a == 0 && rev_;
       if (a == 1) {
         A.Sa = N_[0];
         A.So = N_[0] * N_[1];
@@ -1079,7 +1081,7 @@ class Sim final : public SimBase {
       Z.Sa = NHP_ * N_[1];
       Z.So = NHP_;
       Z.x_blocks = (int)((NH_ + spec_[1].lpw - 1) / spec_[1].lpw);
-      Z.swz = 2 * spec_[1].lpw * (int)sizeof(T) < 128;
+      Z.swz = tile_order(spec_[1].lpw, sizeof(T), 0, Z.x_blocks, large_);
       Z.axis = 2;
       Z.Ny = (int)N_[1];
       Z.Nz = (int)N_[2];
@@ -1108,6 +1110,7 @@ class Sim final : public SimBase {
     plane_args_.p = p_.as<T>();
     plane_args_.nhp = (int)NHP_;
     ca_.nhp = (int)NHP_;
+    ca_.rev = rev_;
     ca_.nl = (int)N_[0];
     ca_.ch = chirp(0);
 
@@ -1452,6 +1455,7 @@ class Sim final : public SimBase {
   DevBuf inv_r_;
   size_t lds_max_ = 65536;   // LDS a workgroup may allocate on this device
   bool large_ = false;       // the fields exceed the last-level cache
+  bool rev_ = false;         // ... twice over: passes turn back (k_dir_pass)
   long long fill_wgs_ = 512;  // workgroups that fill the device (two per CU)
   double c_ref_ = 0, tau_ = 0, y_ = 0, anp_ = 0, d_[3] = {1, 1, 1};
   std::vector<long long> psrc_idx_h_;

@@ -32,7 +32,7 @@ struct ElArgs {
   int Nx;
   long long Sa, So;
   int n_lines, x_blocks;
-  int swz;             // strided: consecutive tiles on one XCD (xcd_wg)
+  int swz;             // strided: order of the workgroups (tile_order)
   int Ny;              // grid extent along y (per-line coordinates)
   int axis;            // axis the lines run along
   int ndim;

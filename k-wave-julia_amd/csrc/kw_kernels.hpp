@@ -45,8 +45,26 @@ __device__ __forceinline__ int xcd_wg(int b, int n) {
 inline bool swizzled_rows(int lpw, int elem_bytes, long long row_pitch_bytes) {
   return 2 * lpw * elem_bytes < 128 || row_pitch_bytes % 128 != 0;
 }
+// On grids larger than the last-level cache (large) with aligned rows, whole
+// rows of tiles (x_blocks of them) go to one XCD, one row after another round
+// the XCDs, so that all of them walk memory together instead of an eighth of
+// the grid apart: 256^3 FP32, y / z pass 105.5 / 104.3 us plain, 103.5 / 103.1 in
+// rows; 512 x 512 x 256 with FP16 maps 398 / 372 and 394 / 365, spectral z pass
+// 133 and 127.5.  Grids in the cache do not care (128^3, 192 x 160 x 128), and
+// unaligned rows prefer the consecutive tiles (240 x 216 x 150: 250 us a step,
+// 252 in rows), as do the spectral y passes (111 us, 113.6).
+// Returns swz: 0 plain order, 1 consecutive tiles on one XCD, else tiles per group.
+inline int tile_order(int lpw, int elem_bytes, long long row_pitch_bytes, int x_blocks, bool large) {
+  if (large && row_pitch_bytes % 128 == 0) return x_blocks > 1 ? x_blocks : 0;
+  return swizzled_rows(lpw, elem_bytes, row_pitch_bytes) ? 1 : 0;
+}
 __device__ __forceinline__ int strided_wg(unsigned b, int swz, unsigned n) {
-  return swz ? xcd_wg((int)b, (int)n) : (int)b;
+  if (swz == 0) return (int)b;
+  if (swz == 1) return xcd_wg((int)b, (int)n);
+  const unsigned g = (unsigned)swz, full = n - n % (8 * g);   // the last groups keep the plain order
+  if (b >= full) return (int)b;
+  const unsigned i = b >> 3;
+  return (int)(((i / g) * 8 + (b & 7)) * g + i % g);
 }
 __device__ __forceinline__ int strided_wg(unsigned b, int swz) { return strided_wg(b, swz, gridDim.x); }
 template <typename T, int N>
@@ -96,7 +114,8 @@ struct PassArgs {
   int n_outer;     // outer count
   int n_lines;     // contiguous: number of real lines
   int x_blocks;    // strided: workgroups along x
-  int swz;         // strided: consecutive tiles on one XCD (xcd_wg)
+  int swz;         // strided: order of the workgroups (tile_order)
+  int rev;         // contiguous: last lines first (k_dir_pass)
   // sources
   SrcList psrc;
   SrcList usrc;
@@ -775,10 +794,20 @@ __device__ __forceinline__ void dir_pass_body(const PassArgs<T>& a, int wg, int 
 // gather of the step before: workgroups from `tiles` on record the rows of r
 // (pressure records only; r.t is that step's index).  As a launch of its own
 // the gather costs 2 us of a 34-us step (512^2 FP32) and 3 of 79 (128^3).
+//
+// Turning back (rev): on grids twice the last-level cache the x pass takes its lines
+// from the last plane to the first, and the spectral y pass
+// that follows goes through the planes from the first, the ones just written;
+// the complex-to-real pass turns back likewise between the inverse y pass and
+// the next step's y pass.  256^3 FP32: spectral y pass 33.0 -> 30.6 us, a step
+// 439.4 -> 434.2; 512 x 512 x 256 with FP16 maps: spectral y pass 111 -> 106.5,
+// complex-to-real 135.8 -> 131.8, a step 1731 -> 1721.  On 240 x 216 x 150, 311
+// MB, the x pass lost more by it (69.4 -> 71.3 us, a step 248.7 -> 250.8), and
+// 128^3, all in the cache, went from 80.2 to 81.7.
 template <typename T, int N, bool CONTIG, bool TWO = false, bool BS = false, int PV = -1>
 __global__ void __launch_bounds__(512) k_dir_pass(PassArgs<T> a, RecArgs<T> r, unsigned tiles) {
   if constexpr (CONTIG) {
-    dir_pass_body<T, N, CONTIG, TWO, BS, PV>(a, (int)blockIdx.x, a.t);
+    dir_pass_body<T, N, CONTIG, TWO, BS, PV>(a, (int)(a.rev ? gridDim.x - 1 - blockIdx.x : blockIdx.x), a.t);
   } else {
     if (blockIdx.x >= tiles) {
       const int j = (int)((blockIdx.x - tiles) * blockDim.x + threadIdx.x);
@@ -845,7 +874,7 @@ struct SpecArgs {
   long long Sa;       // stride along the line (complex elements)
   long long So;       // outer stride
   int x_blocks;
-  int swz;            // consecutive tiles on one XCD (xcd_wg)
+  int swz;            // order of the workgroups (tile_order)
   int mode;           // 0 fwd, 1 inv, 2 fwd*M*inv, 3 fwd*W*inv (1-D window W along the line)
   const T* W;         // mode 3 window (length N, 1/N folded in)
   // octant table addressing: index = kx + MH1*(|line index| + MH2*|outer index|)
@@ -1032,6 +1061,7 @@ struct C2RArgs {
   const Cx<T>* tw;
   T* p;
   int n_lines;
+  int rev;           // last lines first (k_dir_pass)
   int nhp;           // half-spectrum row pitch
   // lines of any length (Bluestein kernels): line length and chirp tables
   int nl;
@@ -1100,7 +1130,7 @@ __device__ __forceinline__ void c2r_body(const C2RArgs<T>& a, int wg) {
 
 template <typename T, int N, bool BS = false, int PV = -1>
 __global__ void __launch_bounds__(256) k_c2r_x(C2RArgs<T> a) {
-  c2r_body<T, N, BS, PV>(a, blockIdx.x);
+  c2r_body<T, N, BS, PV>(a, (int)(a.rev ? gridDim.x - 1 - blockIdx.x : blockIdx.x));
 }
 
 template <typename T, int N>
@@ -1455,7 +1485,7 @@ struct AdjArgs {
   int Nx;
   long long Sa, So;
   int n_lines, x_blocks;
-  int swz;          // strided: consecutive tiles on one XCD (xcd_wg)
+  int swz;          // strided: order of the workgroups (tile_order)
   int accumulate;   // 0: Pb = contribution, 1: Pb += contribution
 };
 
