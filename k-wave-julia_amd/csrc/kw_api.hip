@@ -731,7 +731,7 @@ class Sim final : public SimBase {
     // small grids (2-D, few lines): fewer lines per workgroup until the launch
     // has two workgroups per CU
     if (!batch_mode_) {
-      const int min_lpw = min_lines(contig, tpl, sizeof(T));
+      const int min_lpw = min_lines(contig, tpl, sizeof(T), bs);
       const long long o = contig ? 1 : std::max<long long>(outer, 1);
       while (lpw / 2 >= min_lpw && ((pairs + lpw - 1) / lpw) * o < fill_wgs_) lpw /= 2;
     }
@@ -765,7 +765,7 @@ class Sim final : public SimBase {
     c.req = lpw;
     while (!batch_mode_ && lpw > 1 && lpw / 2 >= NH_) lpw /= 2;
     if (!batch_mode_) {   // as in pass_cfg: fill the device on small grids
-      const int min_lpw = min_lines(false, tpl, sizeof(T));
+      const int min_lpw = min_lines(false, tpl, sizeof(T), bs_[cls == TC_SPEC_Y ? 1 : 2]);
       while (lpw / 2 >= min_lpw && ((NH_ + lpw - 1) / lpw) * std::max<long long>(outer, 1) < fill_wgs_) lpw /= 2;
     }
     c.lpw = lpw;

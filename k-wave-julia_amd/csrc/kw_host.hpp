@@ -272,10 +272,14 @@ struct PassCfg {
 };
 
 // Fewest lines per workgroup a pass on a small grid is split to: one wave, and
-// for strided passes rows of 32 bytes.
-inline int min_lines(bool contig, int tpl, int elem_bytes) {
+// for strided passes rows of 16 bytes, or of 8 on chirp-z lines, whose longer
+// chain of transforms gains more from another CU.  Such grids sit in the L2s,
+// where narrow rows cost issue slots only.  A step of 512 x 512 FP32: 33.8 us at
+// 32 bytes, 32.1 at 16, 32.9 at 8; a call on 300 x 251 FP32 (chirp-z y lines)
+// 25.5 ms, 23.7 and 22.9.
+inline int min_lines(bool contig, int tpl, int elem_bytes, bool chirp = false) {
   const int wave = std::max(1, 64 / tpl);
-  return contig ? wave : std::max(wave, 32 / (2 * elem_bytes));
+  return contig ? wave : std::max(wave, (chirp ? 8 : 16) / (2 * elem_bytes));
 }
 
 // Lines per workgroup of a line pass: 256 threads on contiguous lines, >= 16
