@@ -349,7 +349,6 @@ class ElasticSim {
     for (long long v : idx)
       if (v < 0 || v >= nvox_) raise(KW_ERR_INVALID, "sensor index out of range");
     upload(sens_idx_, idx);
-    zeros(p_);
     auto fill_t = [&](DevBuf& b, long long n, double v) { upload(b, std::vector<T>(n, (T)v)); };
     auto fill_d = [&](DevBuf& b, long long n, double v) { upload(b, std::vector<double>(n, v)); };
     if (rec_ & KW_REC_P) fill_t(p_ts_, nsens_ * Nt_, 0.0);
@@ -367,7 +366,6 @@ class ElasticSim {
     if (rec_ & KW_REC_I_AVG) fill_d(I_avg_, nsens_, 0.0);
     if (rec_ & KW_REC_I_MAX) fill_d(I_max_, nsens_, -INFINITY);
     ra_ = RecArgs<T>{};
-    ra_.p = p_.as<T>();
     for (int a = 0; a < 3; ++a) ra_.u[a] = a < nd_ ? v_[a].template as<T>() : nullptr;
     ra_.ndim = nd_;
     ra_.idx = sens_idx_.as<long long>();
@@ -504,10 +502,8 @@ class ElasticSim {
     if (nsens_ > 0 && !cartesian_) {
       ra_.t = t;
       timed(CLS_RECORD, [&] {
-        HIPC(launch_el_sensor_p<T>(stream_, p_.as<T>(), sn_[0].template as<T>(), sn_[1].template as<T>(),
-                                   nd_ == 3 ? sn_[2].template as<T>() : nullptr, sens_idx_.as<long long>(),
-                                   (int)nsens_, nd_));
-        HIPC(launch_record<T>((unsigned)((nsens_ + 255) / 256), stream_, ra_));
+        HIPC(launch_el_record<T>(stream_, ra_, sn_[0].template as<T>(), sn_[1].template as<T>(),
+                                 nd_ == 3 ? sn_[2].template as<T>() : nullptr));
       });
     }
     t_ = t;
@@ -530,7 +526,7 @@ class ElasticSim {
   bool finalized_ = false, cartesian_ = false;
   size_t lds_max_ = 65536;
   long long fill_wgs_ = 512;
-  DevBuf v_[3], sn_[3], ss_[3], scr_[2], p_;
+  DevBuf v_[3], sn_[3], ss_[3], scr_[2];
   DevBuf lam_, mu_, rho_;
   double lam_s_ = 0, mu_s_ = 0, rho_s_ = 1, kp_ = 1, ks_ = 1;
   DevBuf tw_[3], Dp_[3], Dm_[3], pml_[3], pmlsg_[3];

@@ -230,16 +230,20 @@ __global__ void __launch_bounds__(512) k_el_pass(ElArgs<T> a) {
   L.store(a.s[0], s);
 }
 
-// p = -(sum of normal stresses) / ndim at the sensor points only
+// Sensor gather: p = -(sum of normal stresses) / ndim and the velocities.  One launch; with p formed by a launch of its
+// own the pair took 9.7 us of a 485-us step (256 x 256 x 128 FP32).
 template <typename T>
-__global__ void __launch_bounds__(256) k_el_sensor_p(T* p, const T* s0, const T* s1, const T* s2,
-                                                      const long long* idx, int n, int ndim) {
+__global__ void __launch_bounds__(256) k_el_record(RecArgs<T> a, const T* s0, const T* s1, const T* s2) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
-  const long long i = idx[j];
+  if (j >= a.n) return;
+  const long long i = a.idx[j];
   T tr = s0[i] + s1[i];
-  if (ndim == 3) tr += s2[i];
-  p[i] = -tr / (T)ndim;
+  if (a.ndim == 3) tr += s2[i];
+  const T pv = -tr / (T)a.ndim;
+  T uv[3] = {(T)0, (T)0, (T)0};
+  if (records_u(a.rec))
+    for (int d = 0; d < a.ndim; ++d) uv[d] = a.u[d][i];
+  record_values<T>(a, j, a.t, pv, uv, a.ndim);
 }
 
 // source values of column col (time-major [col][n]) added to / written over f[idx]

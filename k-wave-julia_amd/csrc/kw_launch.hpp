@@ -148,8 +148,7 @@ hipError_t launch_adj_small(int which, hipStream_t s, const void* const* p, cons
 template <typename T>
 hipError_t launch_el(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const ElArgs<T>& a);
 template <typename T>
-hipError_t launch_el_sensor_p(hipStream_t s, T* p, const T* s0, const T* s1, const T* s2, const long long* idx, int n,
-                              int ndim);
+hipError_t launch_el_record(hipStream_t s, const RecArgs<T>& a, const T* s0, const T* s1, const T* s2);
 template <typename T>
 hipError_t launch_el_inject(hipStream_t s, T* f, const long long* idx, const T* vals, int n, int dirichlet);
 

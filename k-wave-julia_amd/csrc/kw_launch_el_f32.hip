@@ -29,11 +29,9 @@ hipError_t launch_el<float>(int n, bool contig, dim3 g, dim3 b, size_t sh, hipSt
 }
 
 template <>
-hipError_t launch_el_sensor_p<float>(hipStream_t s, float* p, const float* s0, const float* s1, const float* s2,
-                                   const long long* idx, int n, int ndim) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL((k_el_sensor_p<float>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, s0, s1, s2, idx, n,
-                     ndim);
+hipError_t launch_el_record<float>(hipStream_t s, const RecArgs<float>& a, const float* s0, const float* s1, const float* s2) {
+  if (a.n <= 0) return hipSuccess;
+  hipLaunchKernelGGL((k_el_record<float>), dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, s, a, s0, s1, s2);
   return hipGetLastError();
 }
 

@@ -29,11 +29,9 @@ hipError_t launch_el<double>(int n, bool contig, dim3 g, dim3 b, size_t sh, hipS
 }
 
 template <>
-hipError_t launch_el_sensor_p<double>(hipStream_t s, double* p, const double* s0, const double* s1, const double* s2,
-                                   const long long* idx, int n, int ndim) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL((k_el_sensor_p<double>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, s0, s1, s2, idx, n,
-                     ndim);
+hipError_t launch_el_record<double>(hipStream_t s, const RecArgs<double>& a, const double* s0, const double* s1, const double* s2) {
+  if (a.n <= 0) return hipSuccess;
+  hipLaunchKernelGGL((k_el_record<double>), dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, s, a, s0, s1, s2);
   return hipGetLastError();
 }
 
