@@ -254,6 +254,15 @@ class ElasticSim {
     cfg_[0] = line_cfg(N_[0], true, N_[1] * N_[2], 0);
     cfg_[1] = line_cfg(N_[1], false, N_[0], N_[2]);
     if (nd_ == 3) cfg_[2] = line_cfg(N_[2], false, N_[0], N_[1]);
+    // Where seven of the fields exceed the last-level cache the FP32 256-point
+    // passes run on 16 threads x 16 elements a line (as the acoustic ones),
+    // except the shear update, which holds three arrays: 256^3, y / z derivative
+    // 38.4 / 43.5 -> 37.2 / 41.0 us, normal stresses 163.7 -> 158.0, a step 945 ->
+    // 917; shear update 67 us, 85 on that plan.  On 256 x 256 x 128 the y derivative
+    // takes 21.1 us on either and the y velocity pass 36 us, 38 on that plan.
+    for (int a = 1; a < nd_; ++a)
+      wide_[a] = sizeof(T) == 4 && N_[a] == 256 && cfg_[a].lpw * plan_tpl(256, kWideFamily) >= 64 &&
+                 beyond_cache(7, N_[0] * N_[1] * N_[2], sizeof(T));
     for (int a = 0; a < nd_; ++a) base_[a] = base_args(a);
 
     build_sources(d);
@@ -419,7 +428,9 @@ class ElasticSim {
   }
   void launch(int axis, const ElArgs<T>& A) {
     const PassCfg& c = cfg_[axis];
-    timed(3 * A.mode + axis, [&] { HIPC(launch_el<T>(c.n, axis == 0, c.grid, c.block, c.shmem, stream_, A)); });
+    const bool wide = axis > 0 && wide_[axis] && A.mode != EL_SHEAR;
+    const dim3 block = wide ? dim3(c.lpw * plan_tpl(c.n, kWideFamily)) : c.block;
+    timed(3 * A.mode + axis, [&] { HIPC(launch_el<T>(c.n, axis == 0, c.grid, block, c.shmem, stream_, A, wide)); });
   }
   // out (+)= D_axis f
   void deriv(int axis, const T* f, const Cx<T>* D, T* out, bool accumulate) {
@@ -531,6 +542,7 @@ class ElasticSim {
   double lam_s_ = 0, mu_s_ = 0, rho_s_ = 1, kp_ = 1, ks_ = 1;
   DevBuf tw_[3], Dp_[3], Dm_[3], pml_[3], pmlsg_[3];
   PassCfg cfg_[3];
+  bool wide_[3] = {false, false, false};   // strided passes but the shear update on the wide-row plan
   ElArgs<T> base_[3];
   // sources
   DevBuf uidx_, uval_[3], sidx_src_, sval_[6];

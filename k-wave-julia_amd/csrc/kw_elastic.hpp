@@ -96,9 +96,11 @@ __device__ __forceinline__ Cx<T> el_med(const LineCtx<T, N, V>& L, const T* m, T
 // MODE is a template parameter so that each epilogue gets its own register
 // allocation (the whole-line loads of the velocity and shear epilogues would
 // otherwise cost the derivative and normal-stress passes occupancy).
-template <typename T, int N, bool CONTIG, int MODE>
+// PV = -1: the pass's default plan family; kWideFamily is instantiated for the
+// FP32 256-point strided passes other than the shear update (large grids).
+template <typename T, int N, bool CONTIG, int MODE, int PV = -1>
 __global__ void __launch_bounds__(512) k_el_pass(ElArgs<T> a) {
-  constexpr int V = default_family<T>(CONTIG ? kC2R : kStrided);
+  constexpr int V = PV >= 0 ? PV : default_family<T>(CONTIG ? kC2R : kStrided);
   constexpr bool OPQ = dir_opaque<T, N, CONTIG, V>();   // as for the acoustic directional passes
   constexpr int E = Plan<N, V>::E;
   constexpr int P = LdsLayout<N>::PITCH;

@@ -145,8 +145,10 @@ hipError_t launch_adj_small(int which, hipStream_t s, const void* const* p, cons
                             int nf = 1);
 
 // Elastic stress-velocity passes and the small per-step kernels around them.
+// wide: on the wide-row plan (FP32 256-point strided passes only)
 template <typename T>
-hipError_t launch_el(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const ElArgs<T>& a);
+hipError_t launch_el(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const ElArgs<T>& a,
+                     bool wide = false);
 template <typename T>
 hipError_t launch_el_record(hipStream_t s, const RecArgs<T>& a, const T* s0, const T* s1, const T* s2);
 template <typename T>

@@ -4,7 +4,18 @@
 namespace kw {
 
 template <>
-hipError_t launch_el<float>(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const ElArgs<float>& a) {
+hipError_t launch_el<float>(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const ElArgs<float>& a,
+                            bool wide) {
+  if (wide) {
+    if (contig || n != 256) return hipErrorInvalidValue;
+    switch (a.mode) {
+      case EL_DERIV: hipLaunchKernelGGL((k_el_pass<float, 256, false, EL_DERIV, kWideFamily>), g, b, sh, s, a); break;
+      case EL_VEL: hipLaunchKernelGGL((k_el_pass<float, 256, false, EL_VEL, kWideFamily>), g, b, sh, s, a); break;
+      case EL_NORMAL: hipLaunchKernelGGL((k_el_pass<float, 256, false, EL_NORMAL, kWideFamily>), g, b, sh, s, a); break;
+      default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+  }
   switch (n) {
 #define M(n_, c_)                                                                            \
   switch (a.mode) {                                                                          \

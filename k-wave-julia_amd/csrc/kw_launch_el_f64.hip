@@ -4,7 +4,9 @@
 namespace kw {
 
 template <>
-hipError_t launch_el<double>(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const ElArgs<double>& a) {
+hipError_t launch_el<double>(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const ElArgs<double>& a,
+                            bool wide) {
+  if (wide) return hipErrorInvalidValue;
   switch (n) {
 #define M(n_, c_)                                                                            \
   switch (a.mode) {                                                                          \
