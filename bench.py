@@ -135,7 +135,7 @@ def cpu_baseline(n_steps_max: int = 20, budget_s: float = 20.0):
 
 def bench_batch(a, tune: bool = True, seq_steps_max: int = 200):
     """64 uneven 2-D firings on 256^2..1024^2 grids; batched (one launch per pass per line
-    length, line lengths on concurrent streams, hipGraph step) against the same simulations
+    length, line lengths on concurrent streams) against the same simulations
     run one after another.  With tune=False the batch runs once, with the default shapes."""
     import numpy as np
     import kwave_amd as K
@@ -198,7 +198,7 @@ def bench_batch(a, tune: bool = True, seq_steps_max: int = 200):
         "warmup": a.warmup, "ms_per_step": (t2 - t1) * 1e3 / a.steps, "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None, "dtype": "f32", "data": "synthetic",
         "config": {"workload": f"batch of {len(sims)} 2D firings, uneven grids {sizes}, heterogeneous c0, "
-                               f"alpha0=0.5 y=1.1, linear array source/sensor, hipGraph step",
+                               f"alpha0=0.5 y=1.1, linear array source/sensor",
                    "voxels_per_step": vox, "parallelism": "single GPU"},
         "sequential_value": sequential, "batched_over_sequential": batched / sequential,
         "untuned_batched_value": vox * a.steps / default_secs, "autotune_s": tune_s,

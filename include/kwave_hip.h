@@ -162,7 +162,8 @@ int32_t kw_ctx_create(int32_t device, kw_ctx** out);
 int32_t kw_ctx_destroy(kw_ctx* ctx);
 
 /* How an axis of length n runs in kw_sim_create (the acoustic solver): 1 on a compiled
- * line-FFT plan, 2 as chirp-z (Bluestein) lines on a power-of-two plan (any length up to
+ * line-FFT plan, 2 on a plan that only single simulations have (33 products of 2, 3 and 5
+ * between 60 and 1000) or as chirp-z (Bluestein) lines on a longer plan (any length up to
  * 2048: 2 to 4x the line-FFT work, the same memory traffic), 0 not at all (n < 1, or longer
  * than 2048 without a plan).  Batches, the adjoint, the elastic solver and the operator entry
  * points take compiled lengths (1) only.  FFTW plans any length (fft_utils.jl:44-62). */

@@ -550,7 +550,7 @@ end
 
 Runs a vector of `(kgrid, medium, source, sensor)` tuples as one batch: every
 pass of the time step is one launch per line length over all simulations and,
-with `use_graph`, one step is one hipGraph replay (`kw_batch_create`);
+with `use_graph`, a step of one grid size is one hipGraph replay (`kw_batch_create`);
 `persistent` selects the persistent-grid launches.  Keyword arguments are
 those of `kspace_first_order` and apply to every simulation; all share
 dimensionality and Nt; time reversal is not batched.

@@ -729,7 +729,8 @@ class Sim final : public SimBase {
     const long long pairs = (lines + 1) / 2;
     while (!batch_mode_ && lpw > 1 && lpw / 2 >= pairs) lpw /= 2;
     // small grids (2-D, few lines): fewer lines per workgroup until the launch
-    // has two workgroups per CU
+    // has two workgroups per CU (filling it to four or eight per CU took 24
+    // firings of 320 x 200 FP32 from 45.5 to 50 us a step)
     if (!batch_mode_) {
       const int min_lpw = min_lines(contig, tpl, sizeof(T), bs);
       const long long o = contig ? 1 : std::max<long long>(outer, 1);
@@ -1473,8 +1474,9 @@ constexpr const char* Sim<T>::kClassNames[];
 // ---------------------------------------------------------------------------
 // Batch of independent simulations: every pass is one launch per line length
 // across all simulations (workgroup -> simulation tables), the step index
-// lives on the device, and one step can be captured in a hipGraph and
-// replayed.  All simulations share precision, dimensionality and Nt.
+// lives on the device, and a step whose passes form one chain can be captured
+// in a hipGraph and replayed (run()).  All simulations share precision,
+// dimensionality and Nt.
 // ---------------------------------------------------------------------------
 struct BatchBase {
   virtual ~BatchBase() = default;

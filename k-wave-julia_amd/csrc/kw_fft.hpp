@@ -763,7 +763,7 @@ __device__ __forceinline__ void line_fft(Cx<T> (&v)[(Plan<N, V>::E)], Cx<T>* lds
 
 // ---------------------------------------------------------------------------
 // Lines of any length n (Bluestein / chirp-z): the DFT of length n as a
-// circular convolution on a compiled power-of-two plan of length N >= 2n - 1.
+// circular convolution on a compiled plan of length N >= 2n - 1.
 //   X_k = c_k sum_j (x_j c_j) d_(k-j),  c_j = exp(-i pi j^2 / n),  d = conj(c)
 //       = c_k IFFT_N( G . FFT_N(c . x) ),  G = FFT_N(g) / N
 // with g_m = d_m (0 <= m < n), g_(N-m) = d_m (0 < m < n), 0 elsewhere; the

@@ -282,9 +282,8 @@ inline int min_lines(bool contig, int tpl, int elem_bytes, bool chirp = false) {
   return contig ? wave : std::max(wave, (chirp ? 8 : 16) / (2 * elem_bytes));
 }
 
-// Lines per workgroup of a line pass: 256 threads on contiguous lines, >= 16
-// line pairs up to 512 threads on strided lines, halved until the lines fit
-// the workgroup's LDS and to the lines that exist.  These passes (elastic,
+// Lines per workgroup of a line pass: contig_lines / strided_lines, halved until
+// the lines fit the workgroup's LDS and to the lines that exist.  These passes (elastic,
 // operator tests) use plan family 2 on contiguous lines.
 // fill_wgs > 0: on small grids, fewer lines per workgroup until the launch has
 // fill_wgs workgroups (keeping one full wave per workgroup).

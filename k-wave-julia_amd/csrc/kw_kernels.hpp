@@ -534,18 +534,21 @@ __device__ __forceinline__ void record_body(const RecArgs<T>& a, int j, int t_in
 // Whether the directional pass keeps each transform's address arithmetic to
 // itself (OPQ in line_fft).  Compiled for gfx950, that never costs the x pass
 // occupancy and raises it (or removes spills) for most lengths; strided
-// passes on 16-element plans (128 ... 4096 points) run at two waves per SIMD
-// either way, and there the merged addresses are faster (512-point strided
-// pass of the 512^3 step: 0.94 ms merged, 1.00 ms separate).
+// passes on 16-element plans run at two waves per SIMD either way, and there
+// the merged addresses are faster (a 512-point strided pass on 32 threads x 16
+// elements, 512^3: 0.94 ms merged, 1.00 ms separate).  A third wave does not
+// help them: with the updates in chunks of 8 elements (168 registers) the 256^3
+// y pass took 109 us, 105 without.
 template <typename T, int N, bool CONTIG, int V>
 constexpr bool dir_opaque() {
   return CONTIG || Plan<N, V>::E != 16;
 }
 
 // Plan families a pass can be launched with besides its default (the
-// autotuner's choice of radix decomposition and threads per line), at 256 and
-// 512 points: 32 x 8 (family 0), 64 x 4 (1) and 32 x 8 (2); 64 x 8.  PV = -1 in a kernel's template arguments selects the
-// pass's default family.
+// autotuner's choice of radix decomposition and threads per line): at 256
+// points 32 x 8 (families 0 and 2) and 64 x 4 (1), at 512 points 64 x 8 in all
+// three.  PV = -1 in a kernel's template arguments selects the pass's default
+// family.
 constexpr bool plan_alternative(int n, int v) {
   return (n == 256 || n == 512) && v >= 0 && v <= 2;
 }

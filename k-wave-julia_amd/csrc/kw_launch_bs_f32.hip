@@ -1,5 +1,5 @@
 // Launchers of the any-length (Bluestein) line passes for float: a line of
-// length n runs on the power-of-two plan n_plan >= 2n - 1 (kw_fft.hpp line_dft).
+// length n runs on the plan n_plan >= 2n - 1 (kw_fft.hpp line_dft).
 #include "kw_launch.hpp"
 
 namespace kw {

@@ -4,7 +4,8 @@ The reference runs one simulation per call; a sweep over transmit elements
 (one firing per simulation) is a loop of calls.  ``kspace_first_order_batch``
 takes that list and runs it through ``kw_batch_*``: each pass of the time
 step is one launch per line length over all simulations, the step index
-lives on the device, and one step is captured in a hipGraph and replayed.
+lives on the device, and a step of one line length is captured in a hipGraph
+and replayed (chains of several line lengths run beside each other on streams).
 With ``persistent`` every batched pass runs as a persistent grid (as many
 workgroups as fit the device at once, each looping over the pass's tiles).
 Results are the same ``SimulationOutput`` objects the single call returns.
