@@ -106,10 +106,11 @@ class Sim final : public SimBase {
 
   void run(long long n) override {
     HIPC(hipSetDevice(dev_));
+    n = std::min(std::max<long long>(n, 0), Nt_ - t_);   // before any sum with t_: n may be the largest int64
     if (line1d_) {
-      run_line1d(std::min(n, Nt_ - t_));
+      run_line1d(n);
     } else {
-      const long long last = std::min(Nt_, t_ + std::max<long long>(n, 0));
+      const long long last = t_ + n;
       while (t_ < last) step(nullptr, t_ + 1 < last);
     }
     HIPC(hipGetLastError());
