@@ -684,12 +684,12 @@ class Sim final : public SimBase {
     // launch geometry
 
     // launch shapes follow the plan length (M_ = N_ unless the axis runs chirp-z lines)
-    cfg_[0] = pass_cfg(M_[0], true, N_[1] * N_[2], 0, TC_DIR_X, bs_[0]);
+    cfg_[0] = pass_cfg(M_[0], true, N_[1] * N_[2], 0, TC_DIR_X);
     if (nd_ > 1) cfg_[1] = pass_cfg(M_[1], false, N_[0], N_[2], TC_DIR_Y);
     if (nd_ > 2) cfg_[2] = pass_cfg(M_[2], false, N_[0], N_[1], TC_DIR_Z);
     if (nd_ > 1) spec_[0] = spec_cfg(M_[1], N_[2], TC_SPEC_Y);
     if (nd_ > 2) spec_[1] = spec_cfg(M_[2], N_[1], TC_SPEC_Z);
-    c2r_ = pass_cfg(M_[0], true, N_[1] * N_[2], 0, TC_C2R, bs_[0]);
+    c2r_ = pass_cfg(M_[0], true, N_[1] * N_[2], 0, TC_C2R);
 
     build_sources(d, het_c);
     build_sensor(d);
@@ -708,8 +708,10 @@ class Sim final : public SimBase {
     return h;
   }
 
-  PassCfg pass_cfg(long long n, bool contig, long long lines, long long outer, int cls, bool bs = false) {
+  PassCfg pass_cfg(long long n, bool contig, long long lines, long long outer, int cls) {
     PassCfg c;
+    // chirp-z lines: their kernels exist in the default family only
+    const bool bs = bs_[cls == TC_DIR_Y ? 1 : (cls == TC_DIR_Z ? 2 : 0)];
     c.n = (int)n;
     // plan family: the pass's default, or a tuned alternative (single simulations on compiled lengths;
     // batch kernels take the defaults)
