@@ -585,6 +585,7 @@ class Sim final : public SimBase {
       if (nd_ != 2) raise(KW_ERR_UNSUPPORTED, "stacked firings need 2-D grids");
       N_[2] = nfire_;
     }
+    const long long x_lines = N_[1] * N_[2];
     for (int a = 0; a < nd_; ++a) {
       if (N_[a] < 1) raise(KW_ERR_INVALID, "grid size must be positive");
       // compiled plan, or a chirp-z (Bluestein) line on a longer plan
@@ -592,7 +593,7 @@ class Sim final : public SimBase {
         raise(KW_ERR_UNSUPPORTED, "axis length " + std::to_string(N_[a]) +
                                       " has no compiled plan; batches take compiled lengths only");
       bs_[a] = !size_supported(N_[a]) && !direct_size(N_[a]);
-      M_[a] = bs_[a] ? bluestein_plan(N_[a]) : N_[a];
+      M_[a] = bs_[a] ? bluestein_plan(N_[a], sizeof(T), a == 0 ? x_lines : 0) : N_[a];
       if (M_[a] == 0)
         raise(KW_ERR_UNSUPPORTED, "axis length " + std::to_string(N_[a]) +
                                       " is longer than the largest chirp-z line (2048) and has no compiled plan");
@@ -715,7 +716,7 @@ class Sim final : public SimBase {
     c.n = (int)n;
     // plan family: the pass's default, or a tuned alternative (single simulations on compiled lengths;
     // batch kernels take the defaults)
-    const int dflt_v = default_family<T>(cls == TC_C2R ? kC2R : (contig ? kContig : kStrided), contig && bs);
+    const int dflt_v = default_family<T>(cls == TC_C2R ? kC2R : (contig ? kContig : kStrided), bs);
     c.pv = (bs || batch_mode_) ? -1 : tuned_plan((int)sizeof(T), cls, (int)n);
     if (c.pv == dflt_v) c.pv = -1;   // the default family: its own kernels
     c.wide = sizeof(T) == 4 && !contig && !bs && large_ && wide_strided((int)n) && (N_[0] * sizeof(T)) % 128 == 0 &&
@@ -735,8 +736,10 @@ class Sim final : public SimBase {
     // has two workgroups per CU (filling it to four or eight per CU took 24
     // firings of 320 x 200 FP32 from 45.5 to 50 us a step)
     if (!batch_mode_) {
-      const int min_lpw = min_lines(contig, tpl, sizeof(T), bs);
       const long long o = contig ? 1 : std::max<long long>(outer, 1);
+      int min_lpw = min_lines(contig, tpl, sizeof(T));
+      // chirp-z lines: narrower still where that leaves half of the CUs without a workgroup
+      if (bs && ((pairs + min_lpw - 1) / min_lpw) * o < fill_wgs_ / 4) min_lpw = min_lines(contig, tpl, sizeof(T), true);
       while (lpw / 2 >= min_lpw && ((pairs + lpw - 1) / lpw) * o < fill_wgs_) lpw /= 2;
     }
     c.lpw = lpw;
@@ -755,10 +758,11 @@ class Sim final : public SimBase {
   PassCfg spec_cfg(long long n, long long outer, int cls) {
     PassCfg c;
     c.n = (int)n;
-    c.pv = (bs_[cls == TC_SPEC_Y ? 1 : 2] || batch_mode_) ? -1 : tuned_plan((int)sizeof(T), cls, (int)n);
-    const int dflt_v = default_family<T>(kStrided);
+    const bool bs = bs_[cls == TC_SPEC_Y ? 1 : 2];
+    c.pv = (bs || batch_mode_) ? -1 : tuned_plan((int)sizeof(T), cls, (int)n);
+    const int dflt_v = default_family<T>(kStrided, bs);
     if (c.pv == dflt_v) c.pv = -1;   // the default family: its own kernels
-    c.wide = sizeof(T) == 4 && !bs_[cls == TC_SPEC_Y ? 1 : 2] && large_ && wide_spectral((int)n) && c.pv < 0;
+    c.wide = sizeof(T) == 4 && !bs && large_ && wide_spectral((int)n) && c.pv < 0;
     const int tpl = plan_tpl((int)n, c.wide ? kWideFamily : (c.pv >= 0 ? c.pv : dflt_v));
     const size_t line_bytes = (size_t)plan_pitch((int)n) * sizeof(Cx<T>);
     int lpw = strided_lines(tpl, sizeof(T), large_);   // one complex line is as wide as a pair of real ones
@@ -769,7 +773,7 @@ class Sim final : public SimBase {
     c.req = lpw;
     while (!batch_mode_ && lpw > 1 && lpw / 2 >= NH_) lpw /= 2;
     if (!batch_mode_) {   // as in pass_cfg: fill the device on small grids
-      const int min_lpw = min_lines(false, tpl, sizeof(T), bs_[cls == TC_SPEC_Y ? 1 : 2]);
+      const int min_lpw = min_lines(false, tpl, sizeof(T), bs);
       while (lpw / 2 >= min_lpw && ((NH_ + lpw - 1) / lpw) * std::max<long long>(outer, 1) < fill_wgs_) lpw /= 2;
     }
     c.lpw = lpw;
@@ -1208,7 +1212,7 @@ class Sim final : public SimBase {
       A.NH = (int)lines;
       A.nl = (int)n;
       A.ch = chirp(a);
-      PassCfg c = line_cfg(M_[a], lines, outer);
+      PassCfg c = line_cfg(M_[a], lines, outer, bs_[a]);
       A.x_blocks = (int)((lines + c.lpw - 1) / c.lpw);
       HIPC(lspec(a, c, A));
       HIPC(hipStreamSynchronize(stream_));
@@ -1247,10 +1251,10 @@ class Sim final : public SimBase {
   }
 
   // launch geometry for complex lines of length n (lines x outer)
-  PassCfg line_cfg(long long n, long long lines, long long outer) {
+  PassCfg line_cfg(long long n, long long lines, long long outer, bool bs) {
     PassCfg c;
     c.n = (int)n;
-    const int tpl = plan_tpl((int)n, default_family<T>(kStrided));
+    const int tpl = plan_tpl((int)n, default_family<T>(kStrided, bs));
     const size_t line_bytes = (size_t)plan_pitch((int)n) * sizeof(Cx<T>);
     int lpw = std::max(1, 256 / tpl);
     while (lpw > 1 && (size_t)lpw * line_bytes > lds_max_) lpw /= 2;

@@ -236,6 +236,7 @@ struct Radices {};
 //   2 / 7  complex-to-real x pass, the adjoint's r2c stage, contiguous elastic
 //          and operator passes in FP32 / FP64,
 //   4      complex-to-real chirp-z lines in FP32,
+//   9      strided and spectral chirp-z lines in FP32,
 //   8      wide rows: strided and spectral passes in FP32 on grids larger than
 //          the last-level cache (kWideFamily below),
 //   5      lines of the fused y-inverse / complex-to-real plane kernel.
@@ -276,6 +277,8 @@ template <int N>
 struct Plan<N, 7> : Plan<N, 3> {};
 template <int N>
 struct Plan<N, 8> : Plan<N, 0> {};
+template <int N>
+struct Plan<N, 9> : Plan<N, 0> {};
 
 // strided and spectral passes
 KW_PLAN(0, 8, 1, 8)
@@ -430,17 +433,22 @@ KW_PLAN(6, 750, 125, 6, 5, 5, 5)
 // complex-to-real (FP64): at most 256 threads
 KW_PLAN(7, 4096, 256, 16, 16, 16)
 // complex-to-real chirp-z lines, which carry the chirp and filter arrays too
-
 KW_PLAN(4, 1024, 128, 8, 8, 4, 4)
 KW_PLAN(4, 2048, 256, 8, 8, 8, 4)
 KW_PLAN(4, 4096, 256, 16, 16, 16)
+// strided and spectral chirp-z lines (FP32): 16 elements a thread spilled 92
+// registers with the chirp beside the fields (256 x 700 FP32 66.9 us a step, 53.1
+// on this plan; 97 x 1013 x 64 640 and 514).  At 4096 points 16 elements stay the
+// faster: 8 leave one line, rows of 8 bytes, to a workgroup of 512 threads (64 x
+// 1500 x 64 512 us, 575).
+KW_PLAN(9, 2048, 256, 8, 8, 8, 4)
 #undef KW_PLAN
 
 enum PassKind { kStrided, kContig, kC2R };
 template <typename T>
 constexpr int default_family(PassKind k, bool chirp = false) {
   if (sizeof(T) == 8) return k == kStrided ? 3 : (k == kContig ? 6 : 7);
-  return k == kStrided ? 0 : (k == kContig ? 1 : (chirp ? 4 : 2));
+  return k == kStrided ? (chirp ? 9 : 0) : (k == kContig ? 1 : (chirp ? 4 : 2));
 }
 
 // Line pairs per workgroup of a strided pass: the largest power of two that

@@ -555,7 +555,7 @@ constexpr bool plan_alternative(int n, int v) {
 
 template <typename T, int N, bool CONTIG, bool TWO = false, bool BS = false, int PV = -1>
 __device__ __forceinline__ void dir_pass_body(const PassArgs<T>& a, int wg, int t_index) {
-  constexpr int V = PV >= 0 ? PV : default_family<T>(CONTIG ? kContig : kStrided, CONTIG && BS);   // plan family
+  constexpr int V = PV >= 0 ? PV : default_family<T>(CONTIG ? kContig : kStrided, BS);   // plan family
   constexpr bool WL = CONTIG && wave_local_lines<N, V>();   // lines inside one wavefront
   constexpr bool OPQ = dir_opaque<T, N, CONTIG, V>();
   constexpr int E = Plan<N, V>::E;
@@ -895,7 +895,7 @@ struct SpecArgs {
 // keeps the plain transforms at a small register footprint.
 template <typename T, int N, int MODE, bool BS = false, int PV = -1>
 __device__ __forceinline__ void spec_pass_body(const SpecArgs<T>& a, int wg) {
-  constexpr int V = PV >= 0 ? PV : default_family<T>(kStrided);   // plan family
+  constexpr int V = PV >= 0 ? PV : default_family<T>(kStrided, BS);   // plan family
   constexpr int TPL = Plan<N, V>::TPL;
   constexpr int E = Plan<N, V>::E;
   constexpr int P = LdsLayout<N>::PITCH;

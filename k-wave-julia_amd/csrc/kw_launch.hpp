@@ -21,9 +21,9 @@
   X(432) X(450) X(480) X(486) X(500) X(540) X(576) X(600) X(648) X(720) X(750) X(800) X(864) X(900) X(960)      \
   X(972) X(1000)
 
-// Plans that carry lines of any other length (Bluestein): powers of two, and
-// 3 and 5 times a power of two between them, so that a line of length n runs
-// on at most 4/3 (2n - 1) points (n = 300: 640 points instead of 1024).
+// Plans that carry lines of any other length (Bluestein): powers of two and,
+// between 64 and 1024, 3 and 5 times a power of two (n = 310: 640 points instead
+// of 1024; n = 513 has 2048 for the 1025 it needs).
 #define KW_BS_SIZES(X) \
   X(8) X(16) X(32) X(64) X(96) X(128) X(192) X(256) X(320) X(384) X(512) X(640) X(768) X(1024) X(2048) X(4096)
 
@@ -35,13 +35,27 @@ bool direct_size(long long n);
 // Plan length of a line of length n without a compiled plan: the smallest
 // n_plan >= 2n - 1 in KW_BS_SIZES, on which its chirp-z transform runs; 0 if n
 // is longer than the largest plan allows (n > 2048).
-inline long long bluestein_plan(long long n) {
+//
+// x_lines > 0: contiguous lines of a grid with that many of them.  Up to 2048
+// (four line pairs a CU) the chain of transforms counts, not the work in it,
+// and the power-of-two plans above 192 and (FP64) 640 points, four elements a
+// thread and no uneven pass, are the faster ones: 70 x 256 FP32 38.8 us a step
+// on 192 points, 28.9 on 256; 1-D 257 FP64 41 on 640, 19.8 on 1024; 257 x 600
+// FP64 83.5 and 61.  With more lines the shorter plan does less work: 257 x 96 x
+// 64 FP64 225 us on 640 points, 240 on 1024; 70 x 200 x 160 FP32 157 on 192, 163
+// on 256.
+inline long long bluestein_plan(long long n, int elem_bytes = 4, long long x_lines = 0) {
   if (n < 1) return 0;
+  long long m = 0;
 #define X(m_) \
-  if (m_ >= 2 * n - 1) return m_;
+  if (m == 0 && m_ >= 2 * n - 1) m = m_;
   KW_BS_SIZES(X)
 #undef X
-  return 0;
+  if (x_lines > 0 && x_lines <= 2048) {
+    if (m == 192) m = 256;
+    if (m == 640 && elem_bytes == 8) m = 1024;
+  }
+  return m;
 }
 // grid of the adjoint's reduction kernels (one partial-sum slot per block)
 inline unsigned adj_reduce_blocks(long long n) {

@@ -55,10 +55,10 @@ int plan_tpl(int n, int family) {
   switch (n) {
 #define X(n_)                                                                                                        \
   case n_: {                                                                                                         \
-    static constexpr int tpl[9] = {Plan<n_, 0>::TPL, Plan<n_, 1>::TPL, Plan<n_, 2>::TPL, Plan<n_, 3>::TPL,            \
+    static constexpr int tpl[10] = {Plan<n_, 0>::TPL, Plan<n_, 1>::TPL, Plan<n_, 2>::TPL, Plan<n_, 3>::TPL,            \
                                    Plan<n_, 4>::TPL, Plan<n_, 5>::TPL, Plan<n_, 6>::TPL, Plan<n_, 7>::TPL,            \
-                                   Plan<n_, 8>::TPL};                                                                \
-    return family >= 0 && family < 9 ? tpl[family] : 0;                                                              \
+                                   Plan<n_, 8>::TPL, Plan<n_, 9>::TPL};                                              \
+    return family >= 0 && family < 10 ? tpl[family] : 0;                                                              \
   }
     KW_SIZES(X)
     KW_DIRECT_SIZES(X)

@@ -37,3 +37,19 @@ def test_long_chirp_z_lines(n, m, form):
             worst = max(rel_l2(out[k], ref[k]) for k in out.keys())
             print(f"    {name} {dtype.__name__} worst rel-L2 {worst:.3e}", flush=True)
             assert worst <= tol, (shape, name, dtype.__name__, worst)
+
+
+@pytest.mark.parametrize("n", [70, 310])
+@pytest.mark.parametrize("lines", [(32, 64), (32, 65)], ids=["2048", "2080"])
+def test_x_lines_on_both_sides_of_the_plan_rule(n, lines):
+    """Up to 2048 x lines 192 points become 256 and (FP64) 640 become 1024; with more they stay."""
+    print(f"\n[case] chirp-z length {n}, {lines[0] * lines[1]} x lines", flush=True)
+    shape = (n,) + lines
+    for name in (ONE, TWO):
+        kg, med, src, sen, kw = scenario(name, shape, seed=n, nt=6)
+        ref = O.kspace_first_order(copy.deepcopy(kg), med, src, sen, **kw)
+        for dtype, tol in ((np.float64, 1e-10), (np.float32, 1e-4)):
+            out = K.kspace_first_order(copy.deepcopy(kg), med, src, sen, data_cast=dtype, **kw)
+            worst = max(rel_l2(out[k], ref[k]) for k in out.keys())
+            print(f"    {name} {dtype.__name__} worst rel-L2 {worst:.3e}", flush=True)
+            assert worst <= tol, (shape, name, dtype.__name__, worst)
