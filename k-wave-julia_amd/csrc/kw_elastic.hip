@@ -254,15 +254,20 @@ class ElasticSim {
     cfg_[0] = line_cfg(N_[0], true, N_[1] * N_[2], 0);
     cfg_[1] = line_cfg(N_[1], false, N_[0], N_[2]);
     if (nd_ == 3) cfg_[2] = line_cfg(N_[2], false, N_[0], N_[1]);
-    // Where seven of the fields exceed the last-level cache the FP32 256-point
-    // passes run on 16 threads x 16 elements a line (as the acoustic ones),
-    // except the shear update, which holds three arrays: 256^3, y / z derivative
-    // 38.4 / 43.5 -> 37.2 / 41.0 us, normal stresses 163.7 -> 158.0, a step 945 ->
-    // 917; shear update 67 us, 85 on that plan.  On 256 x 256 x 128 the y derivative
-    // takes 21.1 us on either and the y velocity pass 36 us, 38 on that plan.
-    for (int a = 1; a < nd_; ++a)
-      wide_[a] = sizeof(T) == 4 && N_[a] == 256 && cfg_[a].lpw * plan_tpl(256, kWideFamily) >= 64 &&
-                 beyond_cache(7, N_[0] * N_[1] * N_[2], sizeof(T));
+    // On grids beyond the last-level cache the strided passes but the shear update,
+    // which holds three arrays (256^3: 67 us, 85 on the wide plan), take the wide-row
+    // plan of lengths that have one (wide_elastic), where rows start on 128-byte
+    // boundaries.  At 256 points it pays from seven fields beyond the cache: 256^3 a
+    // step of 945 us on 32 x 8, 931 on it, 256 x 256 x 128 the other way round (the y
+    // velocity pass 36 us, 38 on it).  Otherwise as strided rows count fields:
+    // 256 x 96 x 320 FP32 539 -> 511 us a step, 256 x 64 x 1024 FP64 2088 -> 1930;
+    // 225 x 320 x 75 FP32, unaligned, 497 on 64 x 5 and 503 on it.
+    for (int a = 1; a < nd_; ++a) {
+      wide_cfg_[a] = cfg_[a];
+      if (wide_elastic<T>((int)N_[a]) && N_[0] * sizeof(T) % 128 == 0 &&
+          beyond_cache(N_[a] == 256 ? 7 : 14, N_[0] * N_[1] * N_[2], sizeof(T)))
+        wide_cfg_[a] = line_cfg(N_[a], false, N_[0], a == 1 ? N_[2] : N_[1], true);
+    }
     for (int a = 0; a < nd_; ++a) base_[a] = base_args(a);
 
     build_sources(d);
@@ -270,19 +275,16 @@ class ElasticSim {
     HIPC(hipStreamSynchronize(stream_));
   }
 
-  PassCfg line_cfg(long long n, bool contig, long long lines, long long outer) {
-    return line_pass_cfg<T>(n, contig, lines, outer, lds_max_, fill_wgs_);
+  PassCfg line_cfg(long long n, bool contig, long long lines, long long outer, bool wide = false) {
+    return line_pass_cfg<T>(n, contig, lines, outer, lds_max_, fill_wgs_, wide);
   }
 
   ElArgs<T> base_args(int axis) {
     ElArgs<T> A{};
-    const PassCfg& c = cfg_[axis];
     A.tw = tw_[axis].template as<Cx<T>>();
     A.Nx = (int)N_[0];
     A.Ny = (int)N_[1];
     A.n_lines = (int)(N_[1] * N_[2]);
-    A.x_blocks = (int)(((N_[0] + 1) / 2 + c.lpw - 1) / c.lpw);
-    A.swz = swizzled_rows(c.lpw, sizeof(T), N_[0] * (long long)sizeof(T));
     if (axis == 0) {
       A.Sa = 1;
       A.So = N_[0];
@@ -426,11 +428,11 @@ class ElasticSim {
     HIPC(hipEventRecord(r.b, stream_));
     prof_->push_back(r);
   }
-  void launch(int axis, const ElArgs<T>& A) {
-    const PassCfg& c = cfg_[axis];
-    const bool wide = axis > 0 && wide_[axis] && A.mode != EL_SHEAR;
-    const dim3 block = wide ? dim3(c.lpw * plan_tpl(c.n, kWideFamily)) : c.block;
-    timed(3 * A.mode + axis, [&] { HIPC(launch_el<T>(c.n, axis == 0, c.grid, block, c.shmem, stream_, A, wide)); });
+  void launch(int axis, ElArgs<T> A) {
+    const PassCfg& c = axis > 0 && A.mode != EL_SHEAR ? wide_cfg_[axis] : cfg_[axis];
+    A.x_blocks = (int)(((N_[0] + 1) / 2 + c.lpw - 1) / c.lpw);
+    A.swz = swizzled_rows(c.lpw, sizeof(T), N_[0] * (long long)sizeof(T));
+    timed(3 * A.mode + axis, [&] { HIPC(launch_el<T>(c.n, axis == 0, c.grid, c.block, c.shmem, stream_, A, c.wide)); });
   }
   // out (+)= D_axis f
   void deriv(int axis, const T* f, const Cx<T>* D, T* out, bool accumulate) {
@@ -542,7 +544,7 @@ class ElasticSim {
   double lam_s_ = 0, mu_s_ = 0, rho_s_ = 1, kp_ = 1, ks_ = 1;
   DevBuf tw_[3], Dp_[3], Dm_[3], pml_[3], pmlsg_[3];
   PassCfg cfg_[3];
-  bool wide_[3] = {false, false, false};   // strided passes but the shear update on the wide-row plan
+  PassCfg wide_cfg_[3];   // strided passes but the shear update: cfg_, or the wide-row plan on large grids
   ElArgs<T> base_[3];
   // sources
   DevBuf uidx_, uval_[3], sidx_src_, sval_[6];

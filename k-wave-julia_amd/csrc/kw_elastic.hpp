@@ -93,11 +93,17 @@ __device__ __forceinline__ Cx<T> el_med(const LineCtx<T, N, V>& L, const T* m, T
   return m ? el_ld(L, m, q) : Cx<T>{s, s};
 }
 
+// Lengths whose strided passes other than the shear update have a wide-row plan.
+template <typename T>
+constexpr bool wide_elastic(int n) {
+  return sizeof(T) == 4 ? n == 256 || n == 320 || n == 1024 : n == 1024;
+}
+
 // MODE is a template parameter so that each epilogue gets its own register
 // allocation (the whole-line loads of the velocity and shear epilogues would
 // otherwise cost the derivative and normal-stress passes occupancy).
 // PV = -1: the pass's default plan family; kWideFamily is instantiated for the
-// FP32 256-point strided passes other than the shear update (large grids).
+// strided passes of wide_elastic lengths other than the shear update (large grids).
 template <typename T, int N, bool CONTIG, int MODE, int PV = -1>
 __global__ void __launch_bounds__(512) k_el_pass(ElArgs<T> a) {
   constexpr int V = PV >= 0 ? PV : default_family<T>(CONTIG ? kC2R : kStrided);

@@ -385,6 +385,7 @@ KW_PLAN(1, 2048, 256, 8, 8, 8, 4)
 KW_PLAN(1, 4096, 512, 8, 8, 8, 8)
 // wide rows
 KW_PLAN(8, 256, 16, 16, 16)
+KW_PLAN(8, 320, 16, 20, 4, 4)
 KW_PLAN(8, 512, 32, 16, 8, 4)
 KW_PLAN(8, 1024, 64, 16, 16, 4)
 // strided and spectral passes (FP64)
@@ -430,6 +431,9 @@ KW_PLAN(6, 600, 100, 6, 10, 10)
 KW_PLAN(6, 640, 64, 10, 8, 8)
 KW_PLAN(6, 648, 108, 6, 12, 9)
 KW_PLAN(6, 750, 125, 6, 5, 5, 5)
+// contiguous elastic passes (FP32): 1024 x 256 x 64, x derivative 48.7 us on 16 x 8
+// x 8, 43.6 on this chain; the complex-to-real pass the same on either (20.2, 20.0)
+KW_PLAN(2, 1024, 64, 16, 16, 4)
 // complex-to-real (FP64): at most 256 threads
 KW_PLAN(7, 4096, 256, 16, 16, 16)
 // complex-to-real chirp-z lines, which carry the chirp and filter arrays too
@@ -479,6 +483,7 @@ constexpr int strided_lines(int tpl, int elem_bytes, bool large = false) {
 constexpr bool beyond_cache(int fields, long long n, int elem_bytes) {
   return (long long)fields * n * elem_bytes > (256LL << 20);
 }
+// (320 points: elastic passes only, wide_elastic.)
 // On such grids the FP32 256-point strided passes and the 256-, 512- and
 // 1024-point spectral passes take 16 elements per thread, which gives 128-byte
 // rows to workgroups of 256 or 512 threads: 512 x 512 x 256, spectral y / z

@@ -287,23 +287,37 @@ inline int min_lines(bool contig, int tpl, int elem_bytes, bool chirp = false) {
 // operator tests) use plan family 2 on contiguous lines.
 // fill_wgs > 0: on small grids, fewer lines per workgroup until the launch has
 // fill_wgs workgroups (keeping one full wave per workgroup).
+// wide: strided lines on the wide-row family.
 template <typename T>
 PassCfg line_pass_cfg(long long n, bool contig, long long lines, long long outer, size_t lds_max,
-                      long long fill_wgs = 0) {
+                      long long fill_wgs = 0, bool wide = false) {
   PassCfg c;
   c.n = (int)n;
-  const int tpl = kw::plan_tpl((int)n, kw::default_family<T>(contig ? kw::kC2R : kw::kStrided));
+  c.wide = wide;
+  const int tpl =
+      kw::plan_tpl((int)n, wide ? kw::kWideFamily : kw::default_family<T>(contig ? kw::kC2R : kw::kStrided));
   const size_t line_bytes = (size_t)kw::plan_pitch((int)n) * sizeof(kw::Cx<T>);
   const long long pairs = (lines + 1) / 2;
   // the elastic solver's nine fields, two partial sums and three maps
   const bool large = !contig && kw::beyond_cache(14, n * lines * std::max<long long>(outer, 1), sizeof(T));
   int lpw = contig ? kw::contig_lines(tpl) : kw::strided_lines(tpl, sizeof(T), large);
   // These passes hold one array and stay below 64 registers, so on large grids
-  // rows of up to 256 bytes pay (256 x 256 x 128 FP32, 128-point z lines: normal
-  // stresses 76.5 -> 69.9 us, velocity 38.2 -> 36.0, a step 486 -> 477.5; FP64 of
-  // 128 x 128 x 256 the same both ways).
-  if (large && 64 % tpl == 0)
-    while (4 * lpw * (int)sizeof(T) <= 256 && 2 * lpw * tpl <= 512) lpw *= 2;
+  // wider rows pay whatever the workgroup's waves: 128 bytes, and 256 where the
+  // lines fill whole waves and rows start on 128-byte boundaries (256 x 256 x 128
+  // FP32, 128-point z lines: normal stresses 76.5 -> 69.9 us, velocity 38.2 -> 36.0;
+  // 256 x 384 x 80, 80-point z lines: normal stresses 114.9 us at 64 bytes, 84.0 at
+  // 128; 256 x 200 x 144, 144-point: 92.5 at 128, a step 491 us, 505 at 256).  Rows
+  // that start anywhere prefer as many lines as 256 threads hold over a power of
+  // two: 243 x 200 x 144, 144-point: normal stresses 145.8 us with 16 lines, 94.8
+  // with 21 (aligned 256 x 200 x 144 the other way round: 92.6 and 114.1).
+  if (large) {
+    const bool aligned = lines * (long long)sizeof(T) % 128 == 0;
+    const int row = aligned && 64 % tpl == 0 ? 256 : 128;
+    if (!aligned && 64 % tpl != 0 && 2 * (256 / tpl) * (int)sizeof(T) >= 128)
+      lpw = 256 / tpl;
+    else
+      while (4 * lpw * (int)sizeof(T) <= row && 2 * lpw * tpl <= 512) lpw *= 2;
+  }
   while (lpw > 1 && (size_t)lpw * line_bytes > lds_max) lpw /= 2;
   while (lpw > 1 && lpw / 2 >= pairs) lpw /= 2;
   {

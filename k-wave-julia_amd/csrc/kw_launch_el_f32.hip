@@ -3,18 +3,30 @@
 
 namespace kw {
 
+// the passes that have a wide-row plan (wide_elastic)
+template <int N>
+static hipError_t el_wide(dim3 g, dim3 b, size_t sh, hipStream_t s, const ElArgs<float>& a) {
+  static_assert(wide_elastic<float>(N), "no wide-row plan");
+  switch (a.mode) {
+    case EL_DERIV: hipLaunchKernelGGL((k_el_pass<float, N, false, EL_DERIV, kWideFamily>), g, b, sh, s, a); break;
+    case EL_VEL: hipLaunchKernelGGL((k_el_pass<float, N, false, EL_VEL, kWideFamily>), g, b, sh, s, a); break;
+    case EL_NORMAL: hipLaunchKernelGGL((k_el_pass<float, N, false, EL_NORMAL, kWideFamily>), g, b, sh, s, a); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
 template <>
 hipError_t launch_el<float>(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const ElArgs<float>& a,
                             bool wide) {
   if (wide) {
-    if (contig || n != 256) return hipErrorInvalidValue;
-    switch (a.mode) {
-      case EL_DERIV: hipLaunchKernelGGL((k_el_pass<float, 256, false, EL_DERIV, kWideFamily>), g, b, sh, s, a); break;
-      case EL_VEL: hipLaunchKernelGGL((k_el_pass<float, 256, false, EL_VEL, kWideFamily>), g, b, sh, s, a); break;
-      case EL_NORMAL: hipLaunchKernelGGL((k_el_pass<float, 256, false, EL_NORMAL, kWideFamily>), g, b, sh, s, a); break;
-      default: return hipErrorInvalidValue;
+    if (contig) return hipErrorInvalidValue;
+    switch (n) {
+      case 256: return el_wide<256>(g, b, sh, s, a);
+      case 320: return el_wide<320>(g, b, sh, s, a);
+      case 1024: return el_wide<1024>(g, b, sh, s, a);
     }
-    return hipGetLastError();
+    return hipErrorInvalidValue;
   }
   switch (n) {
 #define M(n_, c_)                                                                            \

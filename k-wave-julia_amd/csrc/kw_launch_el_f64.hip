@@ -3,10 +3,29 @@
 
 namespace kw {
 
+// the passes that have a wide-row plan (wide_elastic)
+template <int N>
+static hipError_t el_wide(dim3 g, dim3 b, size_t sh, hipStream_t s, const ElArgs<double>& a) {
+  static_assert(wide_elastic<double>(N), "no wide-row plan");
+  switch (a.mode) {
+    case EL_DERIV: hipLaunchKernelGGL((k_el_pass<double, N, false, EL_DERIV, kWideFamily>), g, b, sh, s, a); break;
+    case EL_VEL: hipLaunchKernelGGL((k_el_pass<double, N, false, EL_VEL, kWideFamily>), g, b, sh, s, a); break;
+    case EL_NORMAL: hipLaunchKernelGGL((k_el_pass<double, N, false, EL_NORMAL, kWideFamily>), g, b, sh, s, a); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
 template <>
 hipError_t launch_el<double>(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const ElArgs<double>& a,
                             bool wide) {
-  if (wide) return hipErrorInvalidValue;
+  if (wide) {
+    if (contig) return hipErrorInvalidValue;
+    switch (n) {
+      case 1024: return el_wide<1024>(g, b, sh, s, a);
+    }
+    return hipErrorInvalidValue;
+  }
   switch (n) {
 #define M(n_, c_)                                                                            \
   switch (a.mode) {                                                                          \
