@@ -92,8 +92,9 @@ class Sim final : public SimBase {
   // stacked along a third, uncoupled axis (maps replicated per firing,
   // source/sensor indices offset by the firing's plane); every pass runs over
   // all firings at once and the EOS transform stays 2-D per firing.
-  Sim(int device, const kw_sim_desc& d, bool batch_mode = false, int nfire = 1)
-      : dev_(device), batch_mode_(batch_mode), nfire_(nfire) {
+  // batch_voxels: of the whole batch this simulation belongs to, 0 for a single one
+  Sim(int device, const kw_sim_desc& d, long long batch_voxels = 0, int nfire = 1)
+      : dev_(device), batch_mode_(batch_voxels > 0), batch_voxels_(batch_voxels), nfire_(nfire) {
     build(d);
   }
   ~Sim() override {
@@ -619,6 +620,7 @@ class Sim final : public SimBase {
     plane_ = nvox_ / nfire_;
     // p, u_d, rho_d, two maps and the half spectrum; a batch's launches mix grids
     large_ = !batch_mode_ && beyond_cache(2 * nd_ + 4, nvox_, (int)sizeof(T));
+    batch_rows_ = batch_mode_ && sizeof(T) == 4 && nd_ == 2 && beyond_cache(2 * nd_ + 4, batch_voxels_, (int)sizeof(T));
     rev_ = !batch_mode_ && beyond_cache(nd_ + 2, nvox_, (int)sizeof(T));
     NH_ = N_[0] / 2 + 1;
     NHP_ = (NH_ + 15) / 16 * 16;  // 128-byte aligned spectrum rows (FP32)
@@ -709,6 +711,12 @@ class Sim final : public SimBase {
     return h;
   }
 
+  // Rows of 128 bytes where 512 threads allow them: on grids beyond the last-level
+  // cache, and in FP32 batches of 2-D grids that are so together, on plans of at most
+  // 8 elements a thread (64 uneven grids of 256^2 to 1024^2 572 -> 559 us a step, 40 of
+  // 512^2 226.6 -> 221, 16 of 768^2, 12 elements, 261 ->
+  // 272; four of 256 x 256 x 64 458 -> 467; 100 of 384 x 320 in FP64 485 -> 556).
+  bool wide_rows(int n, int tpl) const { return large_ || (batch_rows_ && n / tpl <= 8); }
   PassCfg pass_cfg(long long n, bool contig, long long lines, long long outer, int cls) {
     PassCfg c;
     // chirp-z lines: their kernels exist in the default family only
@@ -723,7 +731,7 @@ class Sim final : public SimBase {
              c.pv < 0;
     const int tpl = plan_tpl((int)n, c.wide ? kWideFamily : (c.pv >= 0 ? c.pv : dflt_v));
     const size_t line_bytes = (size_t)plan_pitch((int)n) * sizeof(Cx<T>);
-    int lpw = contig ? contig_lines(tpl) : strided_lines(tpl, sizeof(T), large_);
+    int lpw = contig ? contig_lines(tpl) : strided_lines(tpl, sizeof(T), wide_rows((int)n, tpl));
     while (lpw > 1 && (size_t)lpw * line_bytes > lds_max_) lpw /= 2;
     int maxl = (cls == TC_C2R ? 256 : 512) / tpl;   // the kernels' launch bounds
     while (maxl > 1 && (size_t)maxl * line_bytes > lds_max_) maxl /= 2;
@@ -765,7 +773,7 @@ class Sim final : public SimBase {
     c.wide = sizeof(T) == 4 && !bs && large_ && wide_spectral((int)n) && c.pv < 0;
     const int tpl = plan_tpl((int)n, c.wide ? kWideFamily : (c.pv >= 0 ? c.pv : dflt_v));
     const size_t line_bytes = (size_t)plan_pitch((int)n) * sizeof(Cx<T>);
-    int lpw = strided_lines(tpl, sizeof(T), large_);   // one complex line is as wide as a pair of real ones
+    int lpw = strided_lines(tpl, sizeof(T), wide_rows((int)n, tpl));   // one complex line is as wide as a pair of real ones
     while (lpw > 1 && (size_t)lpw * line_bytes > lds_max_) lpw /= 2;
     int maxl = 512 / tpl;
     while (maxl > 1 && (size_t)maxl * line_bytes > lds_max_) maxl /= 2;
@@ -1417,6 +1425,7 @@ class Sim final : public SimBase {
 
   int dev_;
   bool batch_mode_ = false;
+  long long batch_voxels_ = 0;
   long long M_[3] = {1, 1, 1};   // line-FFT plan length per axis (N_, or the chirp-z plan)
   bool bs_[3] = {false, false, false};   // axis runs chirp-z (Bluestein) lines
   DevBuf chc_[3], chf_[3], chb_[3];       // chirp tables of those axes
@@ -1463,6 +1472,7 @@ class Sim final : public SimBase {
   DevBuf inv_r_;
   size_t lds_max_ = 65536;   // LDS a workgroup may allocate on this device
   bool large_ = false;       // the fields exceed the last-level cache
+  bool batch_rows_ = false;  // the batch's do (wide_rows)
   bool rev_ = false;         // ... twice over: passes turn back (k_dir_pass)
   long long fill_wgs_ = 512;  // workgroups that fill the device (two per CU)
   double c_ref_ = 0, tau_ = 0, y_ = 0, anp_ = 0, d_[3] = {1, 1, 1};
@@ -1505,11 +1515,17 @@ class Batch final : public BatchBase {
       cus_ = std::max(cus_, 1);
     }
     if (n < 1) raise(KW_ERR_INVALID, "empty batch");
+    long long voxels = 0;
+    for (int i = 0; i < n; ++i) {
+      long long v = 1;
+      for (int a = 0; a < std::min(descs[i].ndim, 3); ++a) v *= std::max<long long>(1, std::min<long long>(descs[i].N[a], 4096));
+      voxels += v;
+    }
     for (int i = 0; i < n; ++i) {
       if (descs[i].ndim != descs[0].ndim) raise(KW_ERR_INVALID, "a batch needs one dimensionality");
       if (descs[i].Nt != descs[0].Nt) raise(KW_ERR_INVALID, "a batch needs one Nt");
       if (descs[i].tr_data && !descs[i].axisymmetric) raise(KW_ERR_UNSUPPORTED, "time reversal is not batched");
-      sims_.emplace_back(new Sim<T>(device, descs[i], true));
+      sims_.emplace_back(new Sim<T>(device, descs[i], voxels));
     }
     Nt_ = descs[0].Nt;
     nd_ = descs[0].ndim;
@@ -1897,7 +1913,7 @@ void autotune(int dev, const kw_sim_desc& d0, int steps) {
       Restore r;
       g_tune_shift = shift;
       g_tune_plan = plan;
-      s.reset(new Sim<T>(dev, d, false));
+      s.reset(new Sim<T>(dev, d));
     }
     s->trial(warm, steps, ms, lp, nn, pv);
   };
@@ -2207,9 +2223,9 @@ int32_t kw_sim_create_firings(kw_ctx* ctx, const kw_sim_desc* descs, int32_t n_f
   stack_firings(descs, n_firings, F);
   std::unique_ptr<kw_sim> s(new kw_sim);
   if (F.d.precision == 4)
-    s->impl.reset(new Sim<float>(ctx->device, F.d, false, n_firings));
+    s->impl.reset(new Sim<float>(ctx->device, F.d, 0, n_firings));
   else if (F.d.precision == 8)
-    s->impl.reset(new Sim<double>(ctx->device, F.d, false, n_firings));
+    s->impl.reset(new Sim<double>(ctx->device, F.d, 0, n_firings));
   else
     raise(KW_ERR_INVALID, "precision must be 4 or 8");
   *out = s.release();
