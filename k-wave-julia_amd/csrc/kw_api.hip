@@ -714,8 +714,8 @@ class Sim final : public SimBase {
   // Rows of 128 bytes where 512 threads allow them: on grids beyond the last-level
   // cache, and in FP32 batches of 2-D grids that are so together, on plans of at most
   // 8 elements a thread (64 uneven grids of 256^2 to 1024^2 572 -> 559 us a step, 40 of
-  // 512^2 226.6 -> 221, 16 of 768^2, 12 elements, 261 ->
-  // 272; four of 256 x 256 x 64 458 -> 467; 100 of 384 x 320 in FP64 485 -> 556).
+  // 512^2 226.6 -> 221).  Other batches are slower so: 16 of 768^2, 12 elements, 261 ->
+  // 272; four of 256 x 256 x 64 458 -> 467; 100 of 384 x 320 in FP64 485 -> 556.
   bool wide_rows(int n, int tpl) const { return large_ || (batch_rows_ && n / tpl <= 8); }
   PassCfg pass_cfg(long long n, bool contig, long long lines, long long outer, int cls) {
     PassCfg c;
@@ -774,6 +774,12 @@ class Sim final : public SimBase {
     const int tpl = plan_tpl((int)n, c.wide ? kWideFamily : (c.pv >= 0 ? c.pv : dflt_v));
     const size_t line_bytes = (size_t)plan_pitch((int)n) * sizeof(Cx<T>);
     int lpw = strided_lines(tpl, sizeof(T), wide_rows((int)n, tpl));   // one complex line is as wide as a pair of real ones
+    // Beyond the cache rows of 64 bytes at least, whatever the waves, but for FP64 plans
+    // of more than 8 elements: 400-point y lines FP32 27 -> 25 us (256 x 400 x 81, a step
+    // 271 -> 267), 500-point 31 -> 27, FP64 768-point z lines 80 -> 65 (256 x 64 x 768, a
+    // step 715 -> 702); FP64 720-point lines, 9 elements, 79 -> 98.
+    while (large_ && 2 * lpw * (int)sizeof(T) < 64 && 2 * lpw * tpl <= 512 && (sizeof(T) == 4 || (int)n / tpl <= 8))
+      lpw *= 2;
     while (lpw > 1 && (size_t)lpw * line_bytes > lds_max_) lpw /= 2;
     int maxl = 512 / tpl;
     while (maxl > 1 && (size_t)maxl * line_bytes > lds_max_) maxl /= 2;
