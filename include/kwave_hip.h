@@ -229,10 +229,13 @@ int32_t kw_sim_profile(kw_sim* sim, int64_t n_steps, int32_t max_classes, int32_
  * the fastest per (precision, pass, line length) in a process-wide table
  * that later kw_sim_create / kw_batch_create calls read.  With n_sims == 1
  * the trials run descs[0] as a single simulation and, for passes whose line
- * length is 256 or 512, also time the alternative plan families 0, 1, 2
- * (radix schedule and threads per line), which single simulations then use;
+ * length is 256 or 512, also time the plan families 0, 1, 2 (256 points: 16
+ * threads x 16 elements a line, 64 x 4, 32 x 8; 512 points: 32 x 16, 64 x 8,
+ * 64 x 8) that are not the pass's own, which single simulations then use;
  * with n_sims > 1 they run the whole array as one batch (kw_batch_create),
  * so the table fits that batch (batches keep the default plan families).
+ * An entry applies to every grid with that pass and length, so tune on the
+ * grid that is run: grids beyond the last-level cache prefer other shapes.
  * kw_tune_export writes the table as text lines "precision pass n lines"
  * with a fifth column "plan" where a plan family other than the pass's
  * default was chosen (*len = its length; buf gets at most cap-1 bytes plus

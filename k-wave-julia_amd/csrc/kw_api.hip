@@ -43,7 +43,8 @@ thread_local int g_tune_plan = kNoTrial;
 // Plan family of a single simulation's pass: the trial's or the table's
 // choice where the line length has alternatives, else -1 (the default).
 int tuned_plan(int prec, int cls, int n) {
-  if (g_tune_shift != kNoTrial) return plan_alternative(n, g_tune_plan) ? g_tune_plan : -1;
+  if (g_tune_shift != kNoTrial)   // 512 points: family 2 is family 1
+    return plan_alternative(n, g_tune_plan) && !(n == 512 && g_tune_plan == 2) ? g_tune_plan : -1;
   std::lock_guard<std::mutex> lk(g_tune_mu);
   auto it = g_tune_pv.find({prec, cls, n});
   return it != g_tune_pv.end() && plan_alternative(n, it->second) ? it->second : -1;
@@ -425,7 +426,7 @@ class Sim final : public SimBase {
         for (int a = 0; a < nd_; ++a) {
           aa[a].accumulate = a > 0 ? 1 : 0;
           HIPC(launch_adj_pass<T>(cfg_[a].n, a == 0, cfg_[a].grid, cfg_[a].block, cfg_[a].shmem, stream_, aa[a],
-                                  cfg_[a].family()));
+                                  cfg_[a].fam));
         }
       }
     }
@@ -469,28 +470,28 @@ class Sim final : public SimBase {
   // Q = K f and Qd = dK/dc_ref f for a real field f (K = F^-1 M1 F)
   void apply_K(const T* f, const T* M2, T* Q, T* Qd) {
     HIPC(launch_r2c<T>(c2r_.n, c2r_.grid, c2r_.block, c2r_.shmem, stream_, f, S1_.as<Cx<T>>(), (int)(N_[1] * N_[2]),
-                       (int)NHP_, tw_[0].as<Cx<T>>(), c2r_.pv));
+                       (int)NHP_, tw_[0].as<Cx<T>>(), c2r_.fam));
     if (!S2_.p) S2_.alloc((size_t)NHP_ * N_[1] * N_[2] * sizeof(Cx<T>));
     if (nd_ == 3) {
       SpecArgs<T> Y = sa_[0];
       Y.mode = 0;
       Y.S2 = nullptr;
-      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].family()));
+      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].fam));
       SpecArgs<T> Z = sa_[1];
       Z.mode = 5;
       Z.S2 = S2_.as<Cx<T>>();
       Z.M2 = M2;
-      HIPC(launch_spec<T>(spec_[1].n, spec_[1].grid, spec_[1].block, spec_[1].shmem, stream_, Z, spec_[1].family()));
+      HIPC(launch_spec<T>(spec_[1].n, spec_[1].grid, spec_[1].block, spec_[1].shmem, stream_, Z, spec_[1].fam));
       Y.mode = 1;
-      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].family()));
+      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].fam));
       Y.S1 = S2_.as<Cx<T>>();
-      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].family()));
+      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].fam));
     } else if (nd_ == 2) {
       SpecArgs<T> Y = sa_[0];
       Y.mode = 5;
       Y.S2 = S2_.as<Cx<T>>();
       Y.M2 = M2;
-      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].family()));
+      HIPC(launch_spec<T>(spec_[0].n, spec_[0].grid, spec_[0].block, spec_[0].shmem, stream_, Y, spec_[0].fam));
     }
     C2RArgs<T> c = ca_;
     c.S2 = nullptr;
@@ -500,17 +501,17 @@ class Sim final : public SimBase {
     if (nd_ == 1) {
       // 1-D: the multipliers are applied in the c2r pass
       HIPC(hipMemcpyAsync(S2_.p, S1_.p, (size_t)NHP_ * sizeof(Cx<T>), hipMemcpyDeviceToDevice, stream_));
-      HIPC(launch_c2r<T>(c2r_.n, c2r_.grid, c2r_.block, c2r_.shmem, stream_, c, c2r_.pv));
+      HIPC(launch_c2r<T>(c2r_.n, c2r_.grid, c2r_.block, c2r_.shmem, stream_, c, c2r_.fam));
       c.S1 = S2_.as<Cx<T>>();
       c.M1 = M2;
       c.p = Qd;
-      HIPC(launch_c2r<T>(c2r_.n, c2r_.grid, c2r_.block, c2r_.shmem, stream_, c, c2r_.pv));
+      HIPC(launch_c2r<T>(c2r_.n, c2r_.grid, c2r_.block, c2r_.shmem, stream_, c, c2r_.fam));
       return;
     }
-    HIPC(launch_c2r<T>(c2r_.n, c2r_.grid, c2r_.block, c2r_.shmem, stream_, c, c2r_.pv));
+    HIPC(launch_c2r<T>(c2r_.n, c2r_.grid, c2r_.block, c2r_.shmem, stream_, c, c2r_.fam));
     c.S1 = S2_.as<Cx<T>>();
     c.p = Qd;
-    HIPC(launch_c2r<T>(c2r_.n, c2r_.grid, c2r_.block, c2r_.shmem, stream_, c, c2r_.pv));
+    HIPC(launch_c2r<T>(c2r_.n, c2r_.grid, c2r_.block, c2r_.shmem, stream_, c, c2r_.fam));
   }
 
   // d/dc_ref [kappa (1 + nabla1)] / N on the octant (heterogeneous branch)
@@ -717,6 +718,16 @@ class Sim final : public SimBase {
   // 512^2 226.6 -> 221).  Other batches are slower so: 16 of 768^2, 12 elements, 261 ->
   // 272; four of 256 x 256 x 64 458 -> 467; 100 of 384 x 320 in FP64 485 -> 556.
   bool wide_rows(int n, int tpl) const { return large_ || (batch_rows_ && n / tpl <= 8); }
+  // Sets the plan of pass class cls on c.n points: the table's family, where the pass
+  // may take one and it names another plan than `own`, else `own`.  Returns its threads a line.
+  int choose_plan(PassCfg& c, int cls, int dflt, int own, bool tunable) {
+    int v = own;
+    c.pv = tunable ? tuned_plan((int)sizeof(T), cls, c.n) : -1;
+    if (c.pv >= 0 && same_plan(c.n, table_family(c.n, c.pv), own)) c.pv = -1;
+    if (c.pv >= 0) v = table_family(c.n, c.pv);
+    c.fam = same_plan(c.n, v, dflt) ? -1 : v;
+    return plan_tpl(c.n, v);
+  }
   PassCfg pass_cfg(long long n, bool contig, long long lines, long long outer, int cls) {
     PassCfg c;
     // chirp-z lines: their kernels exist in the default family only
@@ -725,11 +736,9 @@ class Sim final : public SimBase {
     // plan family: the pass's default, or a tuned alternative (single simulations on compiled lengths;
     // batch kernels take the defaults)
     const int dflt_v = default_family<T>(cls == TC_C2R ? kC2R : (contig ? kContig : kStrided), bs);
-    c.pv = (bs || batch_mode_) ? -1 : tuned_plan((int)sizeof(T), cls, (int)n);
-    if (c.pv == dflt_v) c.pv = -1;   // the default family: its own kernels
-    c.wide = sizeof(T) == 4 && !contig && !bs && large_ && wide_strided((int)n) && (N_[0] * sizeof(T)) % 128 == 0 &&
-             c.pv < 0;
-    const int tpl = plan_tpl((int)n, c.wide ? kWideFamily : (c.pv >= 0 ? c.pv : dflt_v));
+    const bool wide =
+        sizeof(T) == 4 && !contig && !bs && large_ && wide_strided((int)n) && (N_[0] * sizeof(T)) % 128 == 0;
+    const int tpl = choose_plan(c, cls, dflt_v, wide ? kWideFamily : dflt_v, !bs && !batch_mode_);
     const size_t line_bytes = (size_t)plan_pitch((int)n) * sizeof(Cx<T>);
     int lpw = contig ? contig_lines(tpl) : strided_lines(tpl, sizeof(T), wide_rows((int)n, tpl));
     while (lpw > 1 && (size_t)lpw * line_bytes > lds_max_) lpw /= 2;
@@ -767,11 +776,9 @@ class Sim final : public SimBase {
     PassCfg c;
     c.n = (int)n;
     const bool bs = bs_[cls == TC_SPEC_Y ? 1 : 2];
-    c.pv = (bs || batch_mode_) ? -1 : tuned_plan((int)sizeof(T), cls, (int)n);
     const int dflt_v = default_family<T>(kStrided, bs);
-    if (c.pv == dflt_v) c.pv = -1;   // the default family: its own kernels
-    c.wide = sizeof(T) == 4 && !bs && large_ && wide_spectral((int)n) && c.pv < 0;
-    const int tpl = plan_tpl((int)n, c.wide ? kWideFamily : (c.pv >= 0 ? c.pv : dflt_v));
+    const bool wide = sizeof(T) == 4 && !bs && large_ && wide_spectral((int)n);
+    const int tpl = choose_plan(c, cls, dflt_v, wide ? kWideFamily : dflt_v, !bs && !batch_mode_);
     const size_t line_bytes = (size_t)plan_pitch((int)n) * sizeof(Cx<T>);
     int lpw = strided_lines(tpl, sizeof(T), wide_rows((int)n, tpl));   // one complex line is as wide as a pair of real ones
     // Beyond the cache rows of 64 bytes at least, whatever the waves, but for FP64 plans
@@ -1253,15 +1260,15 @@ class Sim final : public SimBase {
   // pass launches on axis a: the compiled-length kernels or their chirp-z form
   hipError_t ldir(int a, const PassCfg& c, const PassArgs<T>& A, const RecArgs<T>* rec = nullptr) {
     return bs_[a] ? launch_dir_bs<T>(c.n, a == 0, c.grid, c.block, c.shmem, stream_, A, rec)
-                  : launch_dir<T>(c.n, a == 0, c.grid, c.block, c.shmem, stream_, A, c.family(), rec);
+                  : launch_dir<T>(c.n, a == 0, c.grid, c.block, c.shmem, stream_, A, c.fam, rec);
   }
   hipError_t lspec(int a, const PassCfg& c, const SpecArgs<T>& A) {
     return bs_[a] ? launch_spec_bs<T>(c.n, c.grid, c.block, c.shmem, stream_, A)
-                  : launch_spec<T>(c.n, c.grid, c.block, c.shmem, stream_, A, c.family());
+                  : launch_spec<T>(c.n, c.grid, c.block, c.shmem, stream_, A, c.fam);
   }
   hipError_t lc2r(const PassCfg& c, const C2RArgs<T>& A) {
     return bs_[0] ? launch_c2r_bs<T>(c.n, c.grid, c.block, c.shmem, stream_, A)
-                  : launch_c2r<T>(c.n, c.grid, c.block, c.shmem, stream_, A, c.pv);
+                  : launch_c2r<T>(c.n, c.grid, c.block, c.shmem, stream_, A, c.fam);
   }
 
   // launch geometry for complex lines of length n (lines x outer)
@@ -1947,9 +1954,9 @@ void autotune(int dev, const kw_sim_desc& d0, int steps) {
     }
     if (shift > 0 && !changed) shrinking = false;   // every class already at one line per workgroup
   }
-  // plan families 0 (strided), 1 (contiguous), 2 (complex-to-real) on every pass
-  // whose line length has them; a class keeps the default unless another
-  // family is faster (a trial reports -1 for a pass left in its default)
+  // the table families on every pass whose line length has them; a class keeps
+  // its own plan unless another is faster (a trial reports -1 for a pass left
+  // in its own, which a family that names the same plan does)
   for (int plan = 0; has_alt && plan <= 2; ++plan)
     for (int shift : {0, 1}) {
       double ms[TC_COUNT];

@@ -448,6 +448,18 @@ KW_PLAN(4, 4096, 256, 16, 16, 16)
 KW_PLAN(9, 2048, 256, 8, 8, 8, 4)
 #undef KW_PLAN
 
+// Threads per line and radix list of a plan in one number.
+template <int... Rs>
+constexpr long long radix_signature(Radices<Rs...>) {
+  long long s = 0;
+  for (int r : {Rs...}) s = 32 * s + r;
+  return s;
+}
+template <int N, int V>
+constexpr long long plan_signature() {
+  return 1024 * radix_signature(typename Plan<N, V>::R{}) + Plan<N, V>::TPL;
+}
+
 enum PassKind { kStrided, kContig, kC2R };
 template <typename T>
 constexpr int default_family(PassKind k, bool chirp = false) {

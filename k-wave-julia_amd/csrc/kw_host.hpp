@@ -264,9 +264,9 @@ struct PassCfg {
   int n = 0;        // line length
   int lpw = 1;      // lines (pairs) per workgroup
   int req = 1;      // lines per workgroup asked for (before shrinking to small grids)
-  int pv = -1;      // plan family (plan_alternative) or -1 for the pass's default
-  bool wide = false;   // the default is the wide-row family (kWideFamily) on this grid
-  int family() const { return wide ? kw::kWideFamily : pv; }   // as the launchers take it
+  int pv = -1;      // table family in force (plan_alternative), -1: the pass's own choice
+  int fam = -1;     // V of the Plan<n, V> it runs, -1 for the default (as the launchers take it)
+  bool wide = false;   // elastic passes: the wide-row family
   dim3 grid, block;
   size_t shmem = 0;
 };

@@ -544,13 +544,20 @@ constexpr bool dir_opaque() {
   return CONTIG || Plan<N, V>::E != 16;
 }
 
-// Plan families a pass can be launched with besides its default (the
-// autotuner's choice of radix decomposition and threads per line): at 256
-// points 32 x 8 (families 0 and 2) and 64 x 4 (1), at 512 points 64 x 8 in all
-// three.  PV = -1 in a kernel's template arguments selects the pass's default
-// family.
-constexpr bool plan_alternative(int n, int v) {
-  return (n == 256 || n == 512) && v >= 0 && v <= 2;
+// Plan families that the autotuner tries and tuning tables name.  The numbers
+// keep the plans they have meant from the first table on, whatever a pass's
+// default is: at 256 points 0 is 16 threads x 16 elements, 1 is 64 x 4 and 2 is
+// 32 x 8, at 512 points 0 is 32 x 16 and 1 and 2 are 64 x 8.
+constexpr bool plan_alternative(int n, int f) {
+  return (n == 256 || n == 512) && f >= 0 && f <= 2;
+}
+// the V of Plan<n, V> that table family f of length n stands for
+constexpr int table_family(int n, int f) { return f == 0 ? kWideFamily : (n == 256 && f == 2 ? 0 : 1); }
+// Kernels of plan V exist beside those of the default D only where the plans differ.
+// PV = -1 in a kernel's template arguments selects the pass's default family.
+template <int N, int V, int D>
+constexpr bool alternative_kernel() {
+  return (V == 1 || V == kWideFamily || (V == 0 && N == 256)) && plan_signature<N, V>() != plan_signature<N, D>();
 }
 
 template <typename T, int N, bool CONTIG, bool TWO = false, bool BS = false, int PV = -1>

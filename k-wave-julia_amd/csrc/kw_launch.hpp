@@ -64,12 +64,14 @@ inline unsigned adj_reduce_blocks(long long n) {
 }
 // threads per line of length n in plan family `family` (0 where n has no plan)
 int plan_tpl(int n, int family);
+// Whether two families are one plan at length n (lengths with alternatives; others by their numbers).
+bool same_plan(int n, int a, int b);
 int plan_pitch(int n);
 
 // Return hipSuccess or the launch error; unsupported lengths give hipErrorInvalidValue.
 template <typename T>
 // rec (strided passes): also records these sensor rows (k_dir_pass).
-// pv: plan family (plan_alternative), -1 for the pass's default.
+// pv: V of the Plan<n, V> the pass runs (256, 512 and, spectral, 1024 points), -1 for the pass's default.
 hipError_t launch_dir(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const PassArgs<T>& a,
                       int pv = -1, const RecArgs<T>* rec = nullptr);
 template <typename T>

@@ -3,20 +3,35 @@
 
 namespace kw {
 
+// the 256- and 512-point passes on another plan than the default
 template <typename T, int N, int PV>
-static hipError_t adj_alt(bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const AdjArgs<T>& a) {
-  if (contig)
-    hipLaunchKernelGGL((k_adj_pass<T, N, true, PV>), g, b, sh, s, a);
-  else
+static hipError_t adj_one(bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const AdjArgs<T>& a) {
+  if (contig) {
+    if constexpr (alternative_kernel<N, PV, default_family<T>(kContig)>()) {
+      hipLaunchKernelGGL((k_adj_pass<T, N, true, PV>), g, b, sh, s, a);
+      return hipGetLastError();
+    }
+  } else if constexpr (alternative_kernel<N, PV, default_family<T>(kStrided)>()) {
     hipLaunchKernelGGL((k_adj_pass<T, N, false, PV>), g, b, sh, s, a);
-  return hipGetLastError();
+    return hipGetLastError();
+  }
+  return hipErrorInvalidValue;
 }
 template <typename T, int N>
 static hipError_t adj_alt(int pv, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const AdjArgs<T>& a) {
   switch (pv) {
-    case 0: return adj_alt<T, N, 0>(contig, g, b, sh, s, a);
-    case 1: return adj_alt<T, N, 1>(contig, g, b, sh, s, a);
-    case 2: return adj_alt<T, N, 2>(contig, g, b, sh, s, a);
+    case 0: return adj_one<T, N, 0>(contig, g, b, sh, s, a);
+    case 1: return adj_one<T, N, 1>(contig, g, b, sh, s, a);
+    case kWideFamily: return adj_one<T, N, kWideFamily>(contig, g, b, sh, s, a);
+  }
+  return hipErrorInvalidValue;
+}
+template <typename T, int N, int PV>
+static hipError_t r2c_one(dim3 g, dim3 b, size_t sh, hipStream_t s, const T* f, Cx<T>* S, int n_lines, int nhp,
+                          const Cx<T>* tw) {
+  if constexpr (alternative_kernel<N, PV, default_family<T>(kC2R)>()) {
+    hipLaunchKernelGGL((k_r2c_x<T, N, PV>), g, b, sh, s, f, S, n_lines, nhp, tw);
+    return hipGetLastError();
   }
   return hipErrorInvalidValue;
 }
@@ -24,24 +39,20 @@ template <typename T, int N>
 static hipError_t r2c_alt(int pv, dim3 g, dim3 b, size_t sh, hipStream_t s, const T* f, Cx<T>* S, int n_lines,
                           int nhp, const Cx<T>* tw) {
   switch (pv) {
-    case 0: hipLaunchKernelGGL((k_r2c_x<T, N, 0>), g, b, sh, s, f, S, n_lines, nhp, tw); break;
-    case 1: hipLaunchKernelGGL((k_r2c_x<T, N, 1>), g, b, sh, s, f, S, n_lines, nhp, tw); break;
-    case 2: hipLaunchKernelGGL((k_r2c_x<T, N, 2>), g, b, sh, s, f, S, n_lines, nhp, tw); break;
-    default: return hipErrorInvalidValue;
+    case 0: return r2c_one<T, N, 0>(g, b, sh, s, f, S, n_lines, nhp, tw);
+    case 1: return r2c_one<T, N, 1>(g, b, sh, s, f, S, n_lines, nhp, tw);
+    case kWideFamily: return r2c_one<T, N, kWideFamily>(g, b, sh, s, f, S, n_lines, nhp, tw);
   }
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 
 template <typename T>
 hipError_t launch_adj_pass(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const AdjArgs<T>& a,
                            int pv) {
-  if constexpr (sizeof(T) == 4)
-    if (pv == kWideFamily && !contig && n == 256) {
-      hipLaunchKernelGGL((k_adj_pass<T, 256, false, kWideFamily>), g, b, sh, s, a);
-      return hipGetLastError();
-    }
-  if (plan_alternative(n, pv))
-    return n == 256 ? adj_alt<T, 256>(pv, contig, g, b, sh, s, a) : adj_alt<T, 512>(pv, contig, g, b, sh, s, a);
+  if (pv >= 0) {
+    if (n == 256) return adj_alt<T, 256>(pv, contig, g, b, sh, s, a);
+    return n == 512 ? adj_alt<T, 512>(pv, contig, g, b, sh, s, a) : hipErrorInvalidValue;
+  }
   switch (n) {
 #define X(n_)                                                             \
   case n_:                                                                \
@@ -59,9 +70,10 @@ hipError_t launch_adj_pass(int n, bool contig, dim3 g, dim3 b, size_t sh, hipStr
 template <typename T>
 hipError_t launch_r2c(int n, dim3 g, dim3 b, size_t sh, hipStream_t s, const T* f, Cx<T>* S, int n_lines, int nhp,
                       const Cx<T>* tw, int pv) {
-  if (plan_alternative(n, pv))
-    return n == 256 ? r2c_alt<T, 256>(pv, g, b, sh, s, f, S, n_lines, nhp, tw)
-                    : r2c_alt<T, 512>(pv, g, b, sh, s, f, S, n_lines, nhp, tw);
+  if (pv >= 0) {
+    if (n == 256) return r2c_alt<T, 256>(pv, g, b, sh, s, f, S, n_lines, nhp, tw);
+    return n == 512 ? r2c_alt<T, 512>(pv, g, b, sh, s, f, S, n_lines, nhp, tw) : hipErrorInvalidValue;
+  }
   switch (n) {
 #define X(n_)                                                                      \
   case n_:                                                                         \

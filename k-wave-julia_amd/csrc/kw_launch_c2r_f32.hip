@@ -3,20 +3,31 @@
 
 namespace kw {
 
+// the 256- and 512-point pass on another plan than the default
+template <int N, int PV>
+static hipError_t c2r_one(dim3 g, dim3 b, size_t sh, hipStream_t s, const C2RArgs<float>& a) {
+  if constexpr (alternative_kernel<N, PV, default_family<float>(kC2R)>()) {
+    hipLaunchKernelGGL((k_c2r_x<float, N, false, PV>), g, b, sh, s, a);
+    return hipGetLastError();
+  }
+  return hipErrorInvalidValue;
+}
 template <int N>
 static hipError_t c2r_alt(int pv, dim3 g, dim3 b, size_t sh, hipStream_t s, const C2RArgs<float>& a) {
   switch (pv) {
-    case 0: hipLaunchKernelGGL((k_c2r_x<float, N, false, 0>), g, b, sh, s, a); break;
-    case 1: hipLaunchKernelGGL((k_c2r_x<float, N, false, 1>), g, b, sh, s, a); break;
-    case 2: hipLaunchKernelGGL((k_c2r_x<float, N, false, 2>), g, b, sh, s, a); break;
-    default: return hipErrorInvalidValue;
+    case 0: return c2r_one<N, 0>(g, b, sh, s, a);
+    case 1: return c2r_one<N, 1>(g, b, sh, s, a);
+    case kWideFamily: return c2r_one<N, kWideFamily>(g, b, sh, s, a);
   }
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 
 template <>
 hipError_t launch_c2r<float>(int n, dim3 g, dim3 b, size_t sh, hipStream_t s, const C2RArgs<float>& a, int pv) {
-  if (plan_alternative(n, pv)) return n == 256 ? c2r_alt<256>(pv, g, b, sh, s, a) : c2r_alt<512>(pv, g, b, sh, s, a);
+  if (pv >= 0) {
+    if (n == 256) return c2r_alt<256>(pv, g, b, sh, s, a);
+    return n == 512 ? c2r_alt<512>(pv, g, b, sh, s, a) : hipErrorInvalidValue;
+  }
   switch (n) {
 #define X(n_)                                                      \
   case n_:                                                         \

@@ -3,17 +3,23 @@
 
 namespace kw {
 
-// the 256- and 512-point passes in an alternative plan family
+// the 256- and 512-point passes on another plan than the default
 template <int N, int PV>
 static hipError_t dir_alt(bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const PassArgs<double>& a,
                           const RecArgs<double>& r, unsigned tiles) {
-  if (contig && a.S2)
-    hipLaunchKernelGGL((k_dir_pass<double, N, true, true, false, PV>), g, b, sh, s, a, r, tiles);
-  else if (contig)
-    hipLaunchKernelGGL((k_dir_pass<double, N, true, false, false, PV>), g, b, sh, s, a, r, tiles);
-  else
+  if (contig) {
+    if constexpr (alternative_kernel<N, PV, default_family<double>(kContig)>()) {
+      if (a.S2)
+        hipLaunchKernelGGL((k_dir_pass<double, N, true, true, false, PV>), g, b, sh, s, a, r, tiles);
+      else
+        hipLaunchKernelGGL((k_dir_pass<double, N, true, false, false, PV>), g, b, sh, s, a, r, tiles);
+      return hipGetLastError();
+    }
+  } else if constexpr (alternative_kernel<N, PV, default_family<double>(kStrided)>()) {
     hipLaunchKernelGGL((k_dir_pass<double, N, false, false, false, PV>), g, b, sh, s, a, r, tiles);
-  return hipGetLastError();
+    return hipGetLastError();
+  }
+  return hipErrorInvalidValue;
 }
 template <int N>
 static hipError_t dir_alt(int pv, bool contig, dim3 g, dim3 b, size_t sh, hipStream_t s, const PassArgs<double>& a,
@@ -21,7 +27,7 @@ static hipError_t dir_alt(int pv, bool contig, dim3 g, dim3 b, size_t sh, hipStr
   switch (pv) {
     case 0: return dir_alt<N, 0>(contig, g, b, sh, s, a, r, tiles);
     case 1: return dir_alt<N, 1>(contig, g, b, sh, s, a, r, tiles);
-    case 2: return dir_alt<N, 2>(contig, g, b, sh, s, a, r, tiles);
+    case kWideFamily: return dir_alt<N, kWideFamily>(contig, g, b, sh, s, a, r, tiles);
   }
   return hipErrorInvalidValue;
 }
@@ -32,7 +38,10 @@ hipError_t launch_dir<double>(int n, bool contig, dim3 g, dim3 b, size_t sh, hip
   const unsigned tiles = g.x;
   const RecArgs<double> r = rec ? *rec : RecArgs<double>{};
   if (rec && !contig) g.x += ((unsigned)r.n + b.x - 1) / b.x;
-  if (plan_alternative(n, pv)) return n == 256 ? dir_alt<256>(pv, contig, g, b, sh, s, a, r, tiles) : dir_alt<512>(pv, contig, g, b, sh, s, a, r, tiles);
+  if (pv >= 0) {
+    if (n == 256) return dir_alt<256>(pv, contig, g, b, sh, s, a, r, tiles);
+    return n == 512 ? dir_alt<512>(pv, contig, g, b, sh, s, a, r, tiles) : hipErrorInvalidValue;
+  }
   switch (n) {
 #define X(n_)                                                                  \
   case n_:                                                                     \

@@ -67,6 +67,32 @@ int plan_tpl(int n, int family) {
   return 0;
 }
 
+// saved tables name plans by these numbers
+static_assert(plan_signature<256, table_family(256, 0)>() == 1024 * radix_signature(Radices<16, 16>{}) + 16 &&
+                  plan_signature<256, table_family(256, 1)>() == 1024 * radix_signature(Radices<4, 4, 4, 4>{}) + 64 &&
+                  plan_signature<256, table_family(256, 2)>() == 1024 * radix_signature(Radices<8, 8, 4>{}) + 32 &&
+                  plan_signature<512, table_family(512, 0)>() == 1024 * radix_signature(Radices<16, 8, 4>{}) + 32 &&
+                  plan_signature<512, table_family(512, 1)>() == 1024 * radix_signature(Radices<8, 8, 8>{}) + 64 &&
+                  plan_signature<512, table_family(512, 2)>() == plan_signature<512, table_family(512, 1)>(),
+              "the plan families of saved tuning tables keep their meaning");
+bool same_plan(int n, int a, int b) {
+  if (a == b) return true;
+  switch (n) {
+#define X(n_)                                                                                                     \
+  case n_: {                                                                                                      \
+    static constexpr long long sig[10] = {plan_signature<n_, 0>(), plan_signature<n_, 1>(), plan_signature<n_, 2>(), \
+                                          plan_signature<n_, 3>(), plan_signature<n_, 4>(), plan_signature<n_, 5>(), \
+                                          plan_signature<n_, 6>(), plan_signature<n_, 7>(), plan_signature<n_, 8>(), \
+                                          plan_signature<n_, 9>()};                                               \
+    return a >= 0 && a < 10 && b >= 0 && b < 10 && sig[a] == sig[b];                                              \
+  }
+    X(256)
+    X(512)
+#undef X
+  }
+  return false;
+}
+
 int plan_pitch(int n) {
   switch (n) {
 #define X(n_) \

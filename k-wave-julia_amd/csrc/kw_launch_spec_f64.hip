@@ -33,7 +33,7 @@ static hipError_t spec_mode(int mode, dim3 g, dim3 b, size_t sh, hipStream_t s, 
   return hipGetLastError();
 }
 
-// the 256- and 512-point spectral passes in an alternative plan family
+// spectral passes on another plan than the default
 template <int N, int PV>
 static hipError_t spec_alt(dim3 g, dim3 b, size_t sh, hipStream_t s, const SpecArgs<double>& a) {
   switch (a.mode) {
@@ -65,17 +65,25 @@ static hipError_t spec_alt(dim3 g, dim3 b, size_t sh, hipStream_t s, const SpecA
 }
 template <int N>
 static hipError_t spec_alt(int pv, dim3 g, dim3 b, size_t sh, hipStream_t s, const SpecArgs<double>& a) {
+  constexpr int D = default_family<double>(kStrided);
   switch (pv) {
-    case 0: return spec_alt<N, 0>(g, b, sh, s, a);
-    case 1: return spec_alt<N, 1>(g, b, sh, s, a);
-    case 2: return spec_alt<N, 2>(g, b, sh, s, a);
+    case 0:
+      if constexpr (alternative_kernel<N, 0, D>()) return spec_alt<N, 0>(g, b, sh, s, a);
+      break;
+    case 1:
+      if constexpr (alternative_kernel<N, 1, D>()) return spec_alt<N, 1>(g, b, sh, s, a);
+      break;
+    case kWideFamily: return spec_alt<N, kWideFamily>(g, b, sh, s, a);
   }
   return hipErrorInvalidValue;
 }
 
 template <>
 hipError_t launch_spec<double>(int n, dim3 g, dim3 b, size_t sh, hipStream_t s, const SpecArgs<double>& a, int pv) {
-  if (plan_alternative(n, pv)) return n == 256 ? spec_alt<256>(pv, g, b, sh, s, a) : spec_alt<512>(pv, g, b, sh, s, a);
+  if (pv >= 0) {
+    if (n == 256) return spec_alt<256>(pv, g, b, sh, s, a);
+    return n == 512 ? spec_alt<512>(pv, g, b, sh, s, a) : hipErrorInvalidValue;
+  }
   switch (n) {
 #define X(n_)   \
   case n_:      \

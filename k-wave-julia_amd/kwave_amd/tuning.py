@@ -4,8 +4,8 @@ The reference tunes its transforms with FFTW.MEASURE when it creates its
 plans (fft_utils.jl:44-62).  Here each pass is a hand-written line-FFT
 kernel with two free choices: the number of lines a workgroup carries and,
 for line lengths 256 and 512, the plan family (the radix schedule and
-threads per line: 0 = the strided passes' plan, 1 = the contiguous x pass's,
-2 = the complex-to-real pass's).  ``autotune`` times the candidates on the
+threads per line: at 256 points 0 is 16 threads x 16 elements, 1 is 64 x 4 and
+2 is 32 x 8; at 512 points 0 is 32 x 16, 1 and 2 are 64 x 8).  ``autotune`` times the candidates on the
 device for a given simulation and keeps the fastest per (precision, pass,
 line length) in the library's process-wide table, which every later single
 simulation reads (batches take the lines per workgroup and the default plan
