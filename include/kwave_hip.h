@@ -215,6 +215,8 @@ int32_t kw_sim_get_sensor(kw_sim* sim, uint32_t field, double* out);
  * Timing support for benchmarks: run n_steps and return the per-kernel-class
  * average device time in milliseconds (HIP events on the sim's stream).
  * names/ms have room for max_classes entries; *n_classes receives the count.
+ * The launches are those of kw_sim_run: a 1-D simulation whose time loop runs in
+ * one workgroup reports that kernel, up to 256 steps per launch.
  */
 int32_t kw_sim_profile(kw_sim* sim, int64_t n_steps, int32_t max_classes, int32_t* n_classes,
                        const char** names, double* ms, int64_t* launches);
@@ -234,6 +236,8 @@ int32_t kw_sim_profile(kw_sim* sim, int64_t n_steps, int32_t max_classes, int32_
  * 64 x 8) that are not the pass's own, which single simulations then use;
  * with n_sims > 1 they run the whole array as one batch (kw_batch_create),
  * so the table fits that batch (batches keep the default plan families).
+ * (A 1-D simulation's time loop runs in one workgroup and has no such choices;
+ * the trials time the passes that its adjoint runs.)
  * An entry applies to every grid with that pass and length, so tune on the
  * grid that is run: grids beyond the last-level cache prefer other shapes.
  * kw_tune_export writes the table as text lines "precision pass n lines"

@@ -232,7 +232,10 @@ class Sim final : public SimBase {
     HIPC(hipSetDevice(dev_));
     Prof pr;
     pr.ev.reserve(64);
-    for (long long i = 0; i < n && t_ < Nt_; ++i) step(&pr);
+    if (line1d_)   // as run() does: many steps per launch
+      run_line1d(std::min(std::max<long long>(n, 0), Nt_ - t_), &pr);
+    else
+      for (long long i = 0; i < n && t_ < Nt_; ++i) step(&pr);
     HIPC(hipStreamSynchronize(stream_));
     std::vector<double> tot(kNumClasses, 0.0);
     std::vector<long long> cnt(kNumClasses, 0);
@@ -267,8 +270,8 @@ class Sim final : public SimBase {
     for (; done < steps && t_ < Nt_; ++done) step(&pr);
     HIPC(hipStreamSynchronize(stream_));
     static const int cls_of[kNumClasses] = {TC_DIR_X, TC_DIR_Y,  TC_DIR_Z, TC_SPEC_Y, TC_SPEC_Z, TC_SPEC_Y,
-                                            TC_SPEC_Y, TC_C2R,    -1,       -1,        -1};
-    static_assert(kNumClasses == 11, "one tuning class (or -1) per pass class");
+                                            TC_SPEC_Y, TC_C2R,    -1,       -1,        -1,        -1};
+    static_assert(kNumClasses == 12, "one tuning class (or -1) per pass class");
     for (int c = 0; c < TC_COUNT; ++c) ms[c] = 0.0;
     for (auto& r : pr.ev) {
       float e = 0.f;
@@ -542,10 +545,11 @@ class Sim final : public SimBase {
   template <typename U>
   friend class Batch;
   enum Cls { C_DIR_X, C_DIR_Y, C_DIR_Z, C_SPEC_Y_FWD, C_SPEC_Z, C_SPEC_Y_INV, C_SPEC_Y, C_C2R, C_REC, C_TR,
-             C_PLANE_C2R, kNumClasses };
+             C_PLANE_C2R, C_LINE1D, kNumClasses };
   static constexpr const char* kClassNames[kNumClasses] = {
       "k_dir_pass_x_eos", "k_dir_pass_y", "k_dir_pass_z", "k_spec_pass_y_fwd", "k_spec_pass_z_mul",
-      "k_spec_pass_y_inv", "k_spec_pass_y_mul", "k_c2r_x", "k_record", "k_tr_inject", "k_plane_c2r"};
+      "k_spec_pass_y_inv", "k_spec_pass_y_mul", "k_c2r_x", "k_record", "k_tr_inject", "k_plane_c2r",
+      "k_line1d"};
   struct ProfRec {
     int cls;
     hipEvent_t a, b;
@@ -1288,7 +1292,7 @@ class Sim final : public SimBase {
   }
 
   // ---- 1-D grids: many steps per launch, in one workgroup -------------------
-  void run_line1d(long long n) {
+  void run_line1d(long long n, Prof* pr = nullptr) {
     Line1dArgs<T> a;
     std::memset(&a, 0, sizeof(a));
     a.x = pa_[0];
@@ -1306,7 +1310,7 @@ class Sim final : public SimBase {
     while (n > 0) {
       a.nsteps = (int)std::min<long long>(n, 256);   // about a millisecond per launch
       a.t0 = (int)t_ + 1;
-      HIPC(launch_line1d<T>((int)M_[0], bs_[0], stream_, a));
+      launch(pr, C_LINE1D, [&] { HIPC(launch_line1d<T>((int)M_[0], bs_[0], stream_, a)); });
       t_ += a.nsteps;
       n -= a.nsteps;
     }
