@@ -311,6 +311,8 @@ typedef struct kw_batch kw_batch;
 int32_t kw_batch_create(kw_ctx* ctx, const kw_sim_desc* descs, int32_t n_sims, int32_t use_graph, kw_batch** out);
 int32_t kw_batch_run(kw_batch* batch, int64_t n_steps);
 int32_t kw_batch_synchronize(kw_batch* batch);
+/* *captured = 1 once a step has been captured in a graph that kw_batch_run replays, else 0 */
+int32_t kw_batch_captured(const kw_batch* batch, int32_t* captured);
 int32_t kw_batch_sensor_shape(kw_batch* batch, int32_t sim, uint32_t field, int64_t* rows, int64_t* cols);
 int32_t kw_batch_get_sensor(kw_batch* batch, int32_t sim, uint32_t field, double* out);
 int32_t kw_batch_get_field(kw_batch* batch, int32_t sim, int32_t which, double* out);

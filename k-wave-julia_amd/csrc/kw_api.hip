@@ -1519,6 +1519,7 @@ struct BatchBase {
   virtual SimBase* sim(int i) = 0;
   virtual int size() const = 0;
   virtual long long steps_done() const = 0;
+  virtual bool captured() const = 0;
 };
 
 template <typename T>
@@ -1601,6 +1602,7 @@ class Batch final : public BatchBase {
     sims_[i]->t_ = t_;
     return sims_[i].get();
   }
+  bool captured() const override { return exec_ != nullptr; }
   int size() const override { return (int)sims_.size(); }
   long long steps_done() const override { return t_; }
 
@@ -2469,6 +2471,14 @@ int32_t kw_batch_run(kw_batch* b, int64_t n_steps) {
   if (!b) raise(KW_ERR_INVALID, "null batch");
   if (n_steps < 0) raise(KW_ERR_INVALID, "negative step count");
   b->impl->run(n_steps);
+  return KW_OK;
+  KW_GUARD_END
+}
+
+int32_t kw_batch_captured(const kw_batch* b, int32_t* captured) {
+  KW_GUARD_BEGIN
+  if (!b || !captured) raise(KW_ERR_INVALID, "null argument");
+  *captured = b->impl->captured() ? 1 : 0;
   return KW_OK;
   KW_GUARD_END
 }

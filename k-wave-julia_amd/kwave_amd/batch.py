@@ -46,6 +46,13 @@ class Batch:
     def synchronize(self) -> None:
         _lib.check(self._lib.kw_batch_synchronize(self._h))
 
+    @property
+    def captured(self) -> bool:
+        """Whether run() replays a captured graph (use_graph, one chain of passes, after the first step)."""
+        v = C.c_int32()
+        _lib.check(self._lib.kw_batch_captured(self._h, C.byref(v)))
+        return bool(v.value)
+
     def sensor(self, i: int, name: str) -> np.ndarray:
         bit = _lib.REC_BITS[name]
         r, c = C.c_int64(), C.c_int64()
