@@ -1134,7 +1134,7 @@ class Sim final : public SimBase {
     // the fused y-inverse / c2r plane pass where the plane fits a workgroup
     plane_c2r_ = nd_ == 3 && !batch_mode_ && !bs_[0] && !bs_[1] && plane_c2r_supported<T>((int)N_[0], (int)N_[1], lds_max_);
     // a 1-D grid whose line and recorder buffers fit a workgroup's LDS
-    const size_t l1 = nd_ == 1 && !batch_mode_ ? line1d_lds_bytes<T>((int)M_[0], bs_[0]) : 0;
+    const size_t l1 = nd_ == 1 && !batch_mode_ ? line1d_lds_bytes<T>((int)M_[0]) : 0;
     line1d_ = l1 > 0 && l1 <= lds_max_;
     std::memset(&plane_args_, 0, sizeof(plane_args_));
     plane_args_.S1 = S1_.as<Cx<T>>();

@@ -34,8 +34,7 @@ hipError_t launch_line1d<double>(int n, bool bs, hipStream_t s, const Line1dArgs
 }
 
 template <>
-size_t line1d_lds_bytes<double>(int n, bool bs) {
-  (void)bs;
+size_t line1d_lds_bytes<double>(int n) {
   switch (n) {
 #define X(n_) \
   case n_:    \

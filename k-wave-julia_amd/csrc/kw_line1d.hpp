@@ -210,6 +210,6 @@ template <typename T>
 hipError_t launch_line1d(int n, bool bs, hipStream_t s, const Line1dArgs<T>& a);
 // LDS that launch needs; 0 where n has no plan
 template <typename T>
-size_t line1d_lds_bytes(int n, bool bs);
+size_t line1d_lds_bytes(int n);
 
 }  // namespace kw
