@@ -302,18 +302,23 @@ PassCfg line_pass_cfg(long long n, bool contig, long long lines, long long outer
   const bool large = !contig && kw::beyond_cache(14, n * lines * std::max<long long>(outer, 1), sizeof(T));
   int lpw = contig ? kw::contig_lines(tpl) : kw::strided_lines(tpl, sizeof(T), large);
   // These passes hold one array and stay below 64 registers, so on large grids
-  // wider rows pay whatever the workgroup's waves: 128 bytes, and 256 where the
-  // lines fill whole waves and rows start on 128-byte boundaries (256 x 256 x 128
-  // FP32, 128-point z lines: normal stresses 76.5 -> 69.9 us, velocity 38.2 -> 36.0;
-  // 256 x 384 x 80, 80-point z lines: normal stresses 114.9 us at 64 bytes, 84.0 at
-  // 128; 256 x 200 x 144, 144-point: 92.5 at 128, a step 491 us, 505 at 256).  Rows
-  // that start anywhere prefer as many lines as 256 threads hold over a power of
-  // two: 243 x 200 x 144, 144-point: normal stresses 145.8 us with 16 lines, 94.8
-  // with 21 (aligned 256 x 200 x 144 the other way round: 92.6 and 114.1).
+  // wider rows pay:
+  //   lines that fill whole waves: 256 bytes where rows start on 128-byte
+  //     boundaries (256 x 256 x 128 FP32, 128-point z lines: normal stresses 76.5 ->
+  //     69.9 us), 128 on the wide-row plans (640 x 256 x 64: velocity 45.9, 52 at 256);
+  //   other lines: 64 bytes (256 x 200 x 144 FP32, 200-point: velocity 44.6 us at 32
+  //     bytes, 37.2 at 64; FP64 no more than that: 31.2 at 64, 36.1 at 128), in FP32
+  //     128 where 384 threads hold them (256 x 384 x 80, 80-point: normal stresses 114.9
+  //     -> 84.0; 243-point lines, 432 threads: shear 41.8 -> 43.8);
+  //   other lines on rows that start anywhere: as many as 256 threads hold over a
+  //     power of two if that makes 128 bytes (243 x 200 x 144 FP32, 144-point: normal
+  //     stresses 145.8 us with 16 lines, 94.8 with 21; aligned 256 x 200 x 144 the
+  //     other way round, 92.6 and 114.1).
   if (large) {
-    const bool aligned = lines * (long long)sizeof(T) % 128 == 0;
-    const int row = aligned && 64 % tpl == 0 ? 256 : 128;
-    if (!aligned && 64 % tpl != 0 && 2 * (256 / tpl) * (int)sizeof(T) >= 128)
+    const bool aligned = lines * (long long)sizeof(T) % 128 == 0, waves = 64 % tpl == 0;
+    int row = waves ? (aligned && !wide ? 256 : 128) : 64;
+    if (!waves && aligned && sizeof(T) == 4 && 16 * tpl <= 384) row = 128;
+    if (!waves && !aligned && 2 * (256 / tpl) * (int)sizeof(T) >= 128)
       lpw = 256 / tpl;
     else
       while (4 * lpw * (int)sizeof(T) <= row && 2 * lpw * tpl <= 512) lpw *= 2;
