@@ -785,11 +785,13 @@ class Sim final : public SimBase {
     const int tpl = choose_plan(c, cls, dflt_v, wide ? kWideFamily : dflt_v, !bs && !batch_mode_);
     const size_t line_bytes = (size_t)plan_pitch((int)n) * sizeof(Cx<T>);
     int lpw = strided_lines(tpl, sizeof(T), wide_rows((int)n, tpl));   // one complex line is as wide as a pair of real ones
-    // Beyond the cache rows of 64 bytes at least, whatever the waves, but for FP64 plans
-    // of more than 8 elements: 400-point y lines FP32 27 -> 25 us (256 x 400 x 81, a step
-    // 271 -> 267), 500-point 31 -> 27, FP64 768-point z lines 80 -> 65 (256 x 64 x 768, a
-    // step 715 -> 702); FP64 720-point lines, 9 elements, 79 -> 98.
-    while (large_ && 2 * lpw * (int)sizeof(T) < 64 && 2 * lpw * tpl <= 512 && (sizeof(T) == 4 || (int)n / tpl <= 8))
+    // Beyond the cache rows of 64 bytes at least, whatever the waves: 400-point y lines
+    // FP32 27 -> 25 us (256 x 400 x 81, a step 271 -> 267), 500-point 31 -> 27, FP64
+    // 768-point z lines 80 -> 65 (256 x 64 x 768, a step 715 -> 702).  Not for FP64 plans
+    // of more than 8 elements (720 points, 79 -> 98), nor for chirp-z lines (FP64 331
+    // points on 768, 200 x 331 x 100: a step 697 us, 736 with them).
+    const bool wider = large_ && !bs && (sizeof(T) == 4 || (int)n / tpl <= 8);
+    while (wider && 2 * lpw * (int)sizeof(T) < 64 && 2 * lpw * tpl <= 512)
       lpw *= 2;
     while (lpw > 1 && (size_t)lpw * line_bytes > lds_max_) lpw /= 2;
     int maxl = 512 / tpl;
