@@ -236,20 +236,21 @@ struct Radices {};
 //   2 / 7  complex-to-real x pass, the adjoint's r2c stage, contiguous elastic
 //          and operator passes in FP32 / FP64,
 //   4      complex-to-real chirp-z lines in FP32,
-//   9      strided and spectral chirp-z lines in FP32,
 //   8      wide rows: strided and spectral passes in FP32 on grids larger than
 //          the last-level cache (kWideFamily below),
+//   9      strided and spectral chirp-z lines in FP32,
 //   5      lines of the fused y-inverse / complex-to-real plane kernel.
 // What bounds the passes is memory, reached with enough waves in flight: the
 // directional passes carry three to five arrays of E elements per thread, so
-// E <= 8 (FP64) ... 10 keeps them at or below 128 VGPRs (four waves per SIMD)
-// and FP64 out of scratch.  With 16 elements the FP64 128-point x pass spilled
-// 796 bytes per lane and took 85 us on 128^3 (now 31), its strided pass 42
-// (20); with 8 threads per line (32-byte pieces of a row per load) the FP32
-// 128-point x pass took 25 us (now 17).  Lengths with several primes take an
-// uneven pass (StockhamPass) rather than more elements: 240 = 5 x 8 x 6 on 48
-// threads.  Both columns of the table were taken from timed sweeps of radix
-// lists and thread counts at 8 M (FP32) and 4 M (FP64) voxels.
+// E <= 8 (FP64) ... 10 leaves FP32 at four waves per SIMD (159 of 222 kernels,
+// three in 53) and FP64 at two or three (147 and 58) with little or no scratch.
+// With 16 elements the FP64 128-point x pass spilled 796 bytes per lane and took
+// 85 us on 128^3 (now 31), its strided pass 42 (20); with 8 threads per line
+// (32-byte pieces of a row per load) the FP32 128-point x pass took 25 us (now
+// 17).  Lengths with several primes take an uneven pass (StockhamPass) rather
+// than more elements: 240 = 5 x 8 x 6 on 48 threads.  Both columns of the table
+// were taken from timed sweeps of radix lists and thread counts at 8 M (FP32)
+// and 4 M (FP64) voxels.
 template <int N, int V = 0>
 struct Plan;
 #define KW_PLAN(V_, N_, TPL_, ...)                 \
@@ -495,12 +496,12 @@ constexpr int strided_lines(int tpl, int elem_bytes, bool large = false) {
 constexpr bool beyond_cache(int fields, long long n, int elem_bytes) {
   return (long long)fields * n * elem_bytes > (256LL << 20);
 }
-// (320 points: elastic passes only, wide_elastic.)
 // On such grids the FP32 256-point strided passes and the 256-, 512- and
 // 1024-point spectral passes take 16 elements per thread, which gives 128-byte
 // rows to workgroups of 256 or 512 threads: 512 x 512 x 256, spectral y / z
 // passes 125 / 145 us with 8 elements and 110 / 133 with 16; 256^3 35.6 / 37.5
-// and 32.9 / 35.1.  The 512-point directional pass keeps 8 (406 us; 433).
+// and 32.9 / 35.1.  The 512-point directional pass keeps 8 (406 us; 433).  The
+// family's 320-point plan is for elastic passes (wide_elastic).
 constexpr int kWideFamily = 8;
 constexpr bool wide_strided(int n) { return n == 256; }
 constexpr bool wide_spectral(int n) { return n == 256 || n == 512 || n == 1024; }

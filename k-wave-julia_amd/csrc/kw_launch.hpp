@@ -40,7 +40,7 @@ bool direct_size(long long n);
 // (four line pairs a CU) the chain of transforms counts, not the work in it,
 // and the power-of-two plans above 192 and (FP64) 640 points, four elements a
 // thread and no uneven pass, are the faster ones: 70 x 256 FP32 38.8 us a step
-// on 192 points, 28.9 on 256; 1-D 257 FP64 41 on 640, 19.8 on 1024; 257 x 600
+// on 192 points, 27.9 on 256; 1-D 257 FP64 41 on 640, 19.8 on 1024; 257 x 600
 // FP64 83.5 and 61.  With more lines the shorter plan does less work: 257 x 96 x
 // 64 FP64 225 us on 640 points, 240 on 1024; 70 x 200 x 160 FP32 157 on 192, 163
 // on 256.
